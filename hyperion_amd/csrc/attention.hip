@@ -11,21 +11,16 @@
 // when those are null, from the cache (the decoder appends the chunk first; it sizes its
 // rings to hold prefix + L positions).
 //
-// One kernel serves prefill and decode, flash-attention style on v_mfma_f32_16x16x32_bf16:
-//  * A workgroup (4 waves) takes a tile of 64 query rows of one kv head - row r is token
-//    r / G, head-in-group r % G (G = H / KVH) - and walks its visible keys in blocks of 32.
-//    A block's K rows and V go through LDS (AttnLds); each wave computes its 16
-//    rows' scores S = Q K^T (Q rows read from LDS), masks them, and updates the online
-//    softmax in fp32: m = running row maximum (log2 domain), l = running sum, O = O * 2^(m_old
-//    - m) + P V, with P rounded to bf16 for the PV MFMAs (written to LDS and read back in the
-//    A-operand layout).
-//  * Decode (one row tile per kv head) splits the keys over several workgroups; each writes
-//    its unnormalised O with m and l to a workspace, and attn_combine_kernel merges them.
-//  * LDS rows are padded by 16 bytes so the 16 rows (or keys, or dims) an operand read
-//    touches start on different banks.
+// This file holds the decode kernel (at most 16 query rows per kv head), the merges of split
+// keys, the cache write and the dispatch; attention_chunk.hip holds the kernel for chunks.
+// Both are flash-attention style on the matrix cores: scores per block of 32 keys, an online
+// softmax in fp32 (m = running row maximum in the log2 domain, l = running sum), O = O *
+// 2^(m_old - m) + P V with P rounded to bf16. Split keys leave unnormalised O with m and l in
+// a workspace, and attn_combine_kernel (decode) or attn_merge_kernel (chunks) merges them.
 #include <algorithm>
 #include <string>
 
+#include "attention.h"
 #include "common.h"
 #include "kernels.h"
 #include "q4_rmsnorm.h"
@@ -37,45 +32,6 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kAttnThreads = 256;
-constexpr uint32_t kRowsPerTile = 64;   // 4 waves x 16 rows
-constexpr uint32_t kKeyBlock = 32;
-constexpr float kLog2e = 1.4426950408889634f;
-
-struct AttnParams {
-    const uint16_t* q;      // [L][H][D]
-    const uint16_t* k;      // [L][KVH][D]: the chunk, or null when it is in the cache
-    const uint16_t* v;
-    const uint16_t* ck;     // [cap][KVH][D]: the cache
-    const uint16_t* cv;
-    uint16_t* out;          // [L][H][D]
-    float* part_o;          // split partials: [splits][L * H][D]
-    float* part_ml;         // [splits][L * H][2]
-    uint32_t L, H, KVH, G, cap, offset, prefix, window;
-    uint32_t splits, keys_per_split;
-    const uint32_t* pos;    // non-null: offset = *pos, read on the device (graph replays)
-    // The decode form with the prepare folded in (L = 1): q is the raw projection; each
-    // wave normalises and rotates its query rows, and the wave whose keys hold the new
-    // token forms its K/V from k_raw/v_raw and writes them to the cache slot.
-    const float2* rope_cs;  // (cos, sin) [positions][D / 2]
-    const uint16_t* q_w;    // [D]
-    const uint16_t* k_w;    // [D]
-    const uint16_t* k_raw;  // [KVH][D]
-    const uint16_t* v_raw;  // [KVH][D], or null: V = v_norm(k_raw)
-    uint16_t* ck_out;       // the cache, written at the new token's slot
-    uint16_t* cv_out;
-    float eps;
-};
-
-// Graph-replay form: the position comes from device memory, the prefix and the split
-// length follow from it as the host computes them (prefix = min(window, offset) with a
-// window, offset without; keys split evenly in whole key blocks over the fixed grid).
-__device__ __forceinline__ void resolve_position(AttnParams& p) {
-    if (p.pos == nullptr) return;
-    p.offset = *p.pos;
-    p.prefix = p.window != 0u ? min(p.window, p.offset) : p.offset;
-    const uint32_t T = p.prefix + p.L;
-    p.keys_per_split = ((T + p.splits - 1u) / p.splits + kKeyBlock - 1u) / kKeyBlock * kKeyBlock;
-}
 
 // Max and sum over the 16 lanes of a row, in the order of the xor butterfly 1, 2, 4, 8.
 __device__ __forceinline__ float row16_max(float v, uint32_t lane) {
@@ -91,23 +47,6 @@ __device__ __forceinline__ float row16_sum(float v, uint32_t lane) {
     v += xor_lanes<4>(v, lane);
     return v + xor_lanes<8>(v, lane);
 }
-
-template <uint32_t D>
-struct AttnLds {
-    static constexpr uint32_t kRow = D * 2u + 16u;           // Q and K rows (bytes)
-    // V: at head_dim 512 rows as loaded, read by transposing reads; below, transposed on the
-    // way in ([d][32 keys], 16-bit writes in an order rotated by the lane), which measured
-    // faster there (1024-token sliding layer 77 against 112 us; 179 against 203 at 512).
-    static constexpr bool kTrV = D >= 512u;
-    static constexpr uint32_t kVRow = D * 2u + 16u;           // V rows (bytes), kTrV
-    static constexpr uint32_t kVtRow = kKeyBlock * 2u + 16u;  // V^T rows, !kTrV
-    static constexpr uint32_t kPRow = kKeyBlock * 2u + 16u;   // P rows
-    static constexpr uint32_t kQ = 0;
-    static constexpr uint32_t kK = kQ + kRowsPerTile * kRow;
-    static constexpr uint32_t kV = kK + kKeyBlock * kRow;
-    static constexpr uint32_t kP = kV + (kTrV ? kKeyBlock * kVRow : D * kVtRow);
-    static constexpr uint32_t kBytes = kP + (kAttnThreads / 64u) * 16u * kPRow;
-};
 
 __device__ __forceinline__ const uint16_t* key_row(const AttnParams& p, const uint16_t* chunk, const uint16_t* cache,
                                                    uint32_t j, uint32_t hk, uint32_t D) {
@@ -135,207 +74,6 @@ __device__ __forceinline__ bf16x8_t v_operand_tr(uint8_t* p, uint32_t row) {
     return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-template <uint32_t D>
-__global__ __launch_bounds__(kAttnThreads) void attn_kernel(AttnParams p) {
-    resolve_position(p);
-    using Lds = AttnLds<D>;
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u;
-    const uint32_t wave = tid >> 6;
-    const uint32_t j16 = lane & 15u;
-    const uint32_t kb = lane >> 4;
-    const uint32_t hk = blockIdx.y;
-    const uint32_t split = blockIdx.z;
-    const uint32_t rows = p.L * p.G;                     // query rows of this kv head
-    // Workgroups are dispatched x first, then z: the second key split takes the tiles in
-    // reverse, so its longest causal halves start first, on the compute units the first
-    // split's short tiles free early.
-    const uint32_t tile = (split & 1u) != 0u ? gridDim.x - 1u - blockIdx.x : blockIdx.x;
-    const uint32_t row0 = tile * kRowsPerTile;           // first row of the tile
-    const uint32_t T = p.prefix + p.L;
-
-    // The tile's token range and the keys any of its rows can see, within this split.
-    const uint32_t t_lo = row0 / p.G;
-    const uint32_t t_hi = (min(row0 + kRowsPerTile, rows) - 1u) / p.G;
-    uint32_t j_begin = split * p.keys_per_split;
-    uint32_t j_end = min(j_begin + p.keys_per_split, T);
-    j_end = min(j_end, p.prefix + t_hi + 1u);                 // causal: keys up to the last query
-    if (p.window != 0u) {
-        // keys at positions > offset + t_lo - window, i.e. j > prefix + t_lo - window
-        const int64_t lo = static_cast<int64_t>(p.prefix) + t_lo - p.window + 1;
-        if (lo > static_cast<int64_t>(j_begin)) j_begin = static_cast<uint32_t>(lo);
-    }
-
-    // Q tile -> LDS: thread t copies 16-byte chunks (row = c / (D/8), chunk c % (D/8)).
-    constexpr uint32_t kChunks = D / 8u;
-    for (uint32_t c = tid; c < kRowsPerTile * kChunks; c += kAttnThreads) {
-        const uint32_t r = c / kChunks;
-        const uint32_t ch = c - r * kChunks;
-        const uint32_t gr = row0 + r;
-        uint4 val = make_uint4(0u, 0u, 0u, 0u);
-        if (gr < rows) {
-            const uint32_t t = gr / p.G;
-            const uint32_t h = hk * p.G + (gr - t * p.G);
-            val = *reinterpret_cast<const uint4*>(p.q + (static_cast<size_t>(t) * p.H + h) * D + ch * 8u);
-        }
-        *reinterpret_cast<uint4*>(lds + Lds::kQ + r * Lds::kRow + ch * 16u) = val;
-    }
-
-    // Per lane: rows 4 kb + i (i < 4) of the wave's 16; O tiles of 16 dims.
-    constexpr uint32_t kDTiles = D / 16u;
-    f32x4_t o[kDTiles];
-#pragma unroll
-    for (uint32_t t = 0; t < kDTiles; ++t) o[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    float m[4], l[4];
-    int32_t qpos[4];   // -1: a padding row (never visible)
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-        m[i] = -__builtin_huge_valf();
-        l[i] = 0.0f;
-        const uint32_t gr = row0 + wave * 16u + 4u * kb + i;
-        qpos[i] = gr < rows ? static_cast<int32_t>(p.offset + gr / p.G) : -1;
-    }
-    const uint8_t* qrow = lds + Lds::kQ + (wave * 16u + j16) * Lds::kRow;   // A operand row (i = j16)
-    uint8_t* prow_w = lds + Lds::kP + wave * 16u * Lds::kPRow;             // this wave's P [16][32]
-
-    // K and V of a key block: thread tid takes chunks tid + 256 u (key c / (D/8), chunk c %
-    // (D/8): coalesced rows). The next block's chunks are loaded into registers while the
-    // current block computes; staging writes the K rows as loaded and V as AttnLds says.
-    constexpr uint32_t kPer = kKeyBlock * kChunks / kAttnThreads;
-    uint4 kn[kPer];
-    uint4 vn[kPer];
-    const auto fetch = [&](uint32_t jb_) {
-        const uint32_t nk_ = min(kKeyBlock, j_end - jb_);
-#pragma unroll
-        for (uint32_t u = 0; u < kPer; ++u) {
-            const uint32_t c = tid + kAttnThreads * u;
-            const uint32_t r = c / kChunks;
-            const uint32_t ch = c - r * kChunks;
-            kn[u] = make_uint4(0u, 0u, 0u, 0u);
-            vn[u] = make_uint4(0u, 0u, 0u, 0u);
-            if (r < nk_) {
-                kn[u] = *reinterpret_cast<const uint4*>(key_row(p, p.k, p.ck, jb_ + r, hk, D) + ch * 8u);
-                vn[u] = *reinterpret_cast<const uint4*>(key_row(p, p.v, p.cv, jb_ + r, hk, D) + ch * 8u);
-            }
-        }
-    };
-    if (j_begin < j_end) fetch(j_begin);
-
-    for (uint32_t jb = j_begin; jb < j_end; jb += kKeyBlock) {
-        const uint32_t nk = min(kKeyBlock, j_end - jb);
-        __syncthreads();   // the previous block's K/V reads are done (and Q is staged)
-#pragma unroll
-        for (uint32_t u = 0; u < kPer; ++u) {
-            const uint32_t c = tid + kAttnThreads * u;
-            const uint32_t r = c / kChunks;
-            const uint32_t ch = c - r * kChunks;
-            *reinterpret_cast<uint4*>(lds + Lds::kK + r * Lds::kRow + ch * 16u) = kn[u];
-            if constexpr (Lds::kTrV) {
-                *reinterpret_cast<uint4*>(lds + Lds::kV + r * Lds::kVRow + ch * 16u) = vn[u];
-            } else {
-                const uint4 vv = vn[u];
-                uint8_t* col = lds + Lds::kV + (ch * 8u) * Lds::kVtRow + r * 2u;
-#pragma unroll
-                for (uint32_t s2 = 0; s2 < 8u; ++s2) {
-                    const uint32_t e = (s2 + lane) & 7u;
-                    const uint32_t d01 = (e & 2u) ? vv.y : vv.x;
-                    const uint32_t d23 = (e & 2u) ? vv.w : vv.z;
-                    const uint32_t dw = (e & 4u) ? d23 : d01;
-                    *reinterpret_cast<uint16_t*>(col + e * Lds::kVtRow) =
-                        static_cast<uint16_t>((e & 1u) ? (dw >> 16) : (dw & 0xFFFFu));
-                }
-            }
-        }
-        __syncthreads();
-        if (jb + kKeyBlock < j_end) fetch(jb + kKeyBlock);   // in flight during this block
-
-        // S = Q K^T for the wave's 16 rows x 32 keys (two column tiles of 16 keys).
-        f32x4_t s[2] = {f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}};
-#pragma unroll 4
-        for (uint32_t st = 0; st < D / 32u; ++st) {
-            const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(qrow + (st * 32u + kb * 8u) * 2u);
-#pragma unroll
-            for (uint32_t c = 0; c < 2; ++c) {
-                const bf16x8_t b = *reinterpret_cast<const bf16x8_t*>(lds + Lds::kK + (16u * c + j16) * Lds::kRow +
-                                                                      (st * 32u + kb * 8u) * 2u);
-                s[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, s[c], 0, 0, 0);
-            }
-        }
-
-        // Mask, online softmax (log2 domain), P -> LDS as bf16.
-#pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) {
-            float sv[2];
-            float bmax = -__builtin_huge_valf();
-#pragma unroll
-            for (uint32_t c = 0; c < 2; ++c) {
-                const uint32_t key = 16u * c + j16;
-                const int32_t kpos = static_cast<int32_t>(p.offset - p.prefix + jb + key);
-                const bool vis = key < nk && qpos[i] >= 0 && kpos <= qpos[i] &&
-                                 (p.window == 0u || kpos > qpos[i] - static_cast<int32_t>(p.window));
-                sv[c] = vis ? s[c][i] * kLog2e : -__builtin_huge_valf();
-                bmax = fmaxf(bmax, sv[c]);
-            }
-            bmax = row16_max(bmax, lane);
-            const float m_new = fmaxf(m[i], bmax);
-            const bool any = m_new > -__builtin_huge_valf();
-            const float alpha = any ? exp2f(m[i] - m_new) : 1.0f;   // m[i] = -inf -> 0
-            float psum = 0.0f;
-#pragma unroll
-            for (uint32_t c = 0; c < 2; ++c) {
-                const float pv = any && sv[c] > -__builtin_huge_valf() ? exp2f(sv[c] - m_new) : 0.0f;
-                psum += pv;
-                *reinterpret_cast<uint16_t*>(prow_w + (4u * kb + i) * Lds::kPRow + (16u * c + j16) * 2u) =
-                    f32_to_bf16_bits(pv);
-            }
-            psum = row16_sum(psum, lane);
-            l[i] = l[i] * alpha + psum;
-            m[i] = any ? m_new : m[i];
-#pragma unroll
-            for (uint32_t t = 0; t < kDTiles; ++t) o[t][i] *= alpha;
-        }
-        // P (16 x 32 keys) as the A operand, V^T as B: O += P V.
-        const bf16x8_t pa = *reinterpret_cast<const bf16x8_t*>(prow_w + j16 * Lds::kPRow + kb * 16u);
-        if constexpr (Lds::kTrV) {
-            uint8_t* vt = lds + Lds::kV + (8u * kb + (j16 >> 2)) * Lds::kVRow + (j16 & 3u) * 8u;
-#pragma unroll
-            for (uint32_t t = 0; t < kDTiles; ++t) {
-                o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, v_operand_tr(vt + 32u * t, Lds::kVRow), o[t], 0, 0, 0);
-            }
-        } else {
-#pragma unroll
-            for (uint32_t t = 0; t < kDTiles; ++t) {
-                const bf16x8_t b = *reinterpret_cast<const bf16x8_t*>(lds + Lds::kV + (16u * t + j16) * Lds::kVtRow + kb * 16u);
-                o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, b, o[t], 0, 0, 0);
-            }
-        }
-    }
-
-    // Rows 4 kb + i of the wave, dims 16 t + j16.
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-        const uint32_t gr = row0 + wave * 16u + 4u * kb + i;
-        if (gr >= rows) continue;
-        const uint32_t t = gr / p.G;
-        const uint32_t h = hk * p.G + (gr - t * p.G);
-        const size_t orow = static_cast<size_t>(t) * p.H + h;   // [L][H] row of the output
-        if (p.splits == 1u) {
-            const float inv = l[i] > 0.0f ? 1.0f / l[i] : 0.0f;
-#pragma unroll
-            for (uint32_t tt = 0; tt < kDTiles; ++tt) p.out[orow * D + 16u * tt + j16] = f32_to_bf16_bits(o[tt][i] * inv);
-        } else {
-            const size_t prow = static_cast<size_t>(split) * p.L * p.H + orow;
-#pragma unroll
-            for (uint32_t tt = 0; tt < kDTiles; ++tt) p.part_o[prow * D + 16u * tt + j16] = o[tt][i];
-            if (j16 == 0u) {
-                p.part_ml[prow * 2u] = m[i];
-                p.part_ml[prow * 2u + 1u] = l[i];
-            }
-        }
-    }
-}
-
 // Decode form (at most 16 query rows per kv head: L * G <= 16, a single MFMA row tile).
 // Each wave is an independent split of the keys, with nothing shared across waves:
 //  * Q stays in registers as the A operand of S = Q K^T for the whole kernel;
@@ -344,7 +82,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_kernel(AttnParams p) {
 //  * V rows load coalesced into the wave's own LDS as they are ([32 keys][d], 16-byte
 //    writes) and reach the B operand of O += P V by transposing reads (two
 //    ds_read_b64_tr_b16 per 16-dim tile: lane (dim j, kb) takes keys 8kb .. 8kb + 7);
-//  * the online softmax, P in bf16 and the P.V products are those of attn_kernel.
+//  * the online softmax and P in bf16 as above.
 // Every split writes its unnormalised rows with (m, l); attn_combine_kernel merges them.
 template <uint32_t D>
 struct DecodeLds {
@@ -814,10 +552,9 @@ __global__ __launch_bounds__(kAttnThreads) void attn_combine_kernel(AttnParams p
     }
 }
 
-// The chunk form's merge of its key splits (at most kChunkMaxSplits): thread c takes the 8
-// dims ch = c % (D/8) of row c / (D/8), the splits weighted as in attn_combine_kernel
-// (2^(m_s - max m), the sum of l_s, the divided sum).
-constexpr uint32_t kChunkMaxSplits = 2;
+// The chunk form's merge of its key splits: thread c takes the 8 dims ch = c % (D/8) of row
+// c / (D/8), the splits weighted as in attn_combine_kernel (2^(m_s - max m), the sum of l_s,
+// the divided sum).
 template <uint32_t D>
 __global__ __launch_bounds__(kAttnThreads) void attn_merge_kernel(AttnParams p) {
     constexpr uint32_t kCh = D / 8u;
@@ -826,29 +563,21 @@ __global__ __launch_bounds__(kAttnThreads) void attn_merge_kernel(AttnParams p) 
     if (c >= rows * kCh) return;
     const uint64_t row = c / kCh;
     const uint32_t ch = static_cast<uint32_t>(c - row * kCh);
-    float ms[kChunkMaxSplits];
-    float ls[kChunkMaxSplits];
-    float4 lo[kChunkMaxSplits];
-    float4 hi[kChunkMaxSplits];
     float mx = -__builtin_huge_valf();
-#pragma unroll
-    for (uint32_t s = 0; s < kChunkMaxSplits; ++s) {
-        const bool live = s < p.splits;
-        ms[s] = live ? p.part_ml[(s * rows + row) * 2u] : -__builtin_huge_valf();
-        ls[s] = live ? p.part_ml[(s * rows + row) * 2u + 1u] : 0.0f;
-        const float4* o4 = reinterpret_cast<const float4*>(p.part_o + (s * rows + row) * D + ch * 8u);
-        lo[s] = live ? o4[0] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        hi[s] = live ? o4[1] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        mx = fmaxf(mx, ms[s]);
-    }
+    for (uint32_t s = 0; s < p.splits; ++s) mx = fmaxf(mx, p.part_ml[(s * rows + row) * 2u]);
     float den = 0.0f;
     float num[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (uint32_t s = 0; s < kChunkMaxSplits; ++s) {
-        const float w = ms[s] == -__builtin_huge_valf() || mx == -__builtin_huge_valf() ? 0.0f : exp2f(ms[s] - mx);
+#pragma unroll 4
+    for (uint32_t s = 0; s < p.splits; ++s) {
+        const float ms = p.part_ml[(s * rows + row) * 2u];
+        const float ls = p.part_ml[(s * rows + row) * 2u + 1u];
+        const float4* o4 = reinterpret_cast<const float4*>(p.part_o + (s * rows + row) * D + ch * 8u);
+        const float4 lo = o4[0];
+        const float4 hi = o4[1];
+        const float w = ms == -__builtin_huge_valf() || mx == -__builtin_huge_valf() ? 0.0f : exp2f(ms - mx);
         if (w == 0.0f) continue;
-        den += w * ls[s];
-        const float v[8] = {lo[s].x, lo[s].y, lo[s].z, lo[s].w, hi[s].x, hi[s].y, hi[s].z, hi[s].w};
+        den += w * ls;
+        const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
         for (int e = 0; e < 8; ++e) num[e] += w * v[e];
     }
@@ -907,61 +636,40 @@ void launch_decode_d(const AttnParams& p, bool prep, hipStream_t stream) {
     HYP_HIP_CHECK(hipGetLastError());
 }
 
-template <uint32_t D>
-void launch_attn_d(const AttnParams& p, hipStream_t stream) {
-    constexpr size_t lds = AttnLds<D>::kBytes;
-    static_assert(lds <= 160u * 1024u, "attention LDS");
-    if (lds > 65536u) {
-        static thread_local int configured_device = -1;
-        int dev = 0;
-        HYP_HIP_CHECK(hipGetDevice(&dev));
-        if (configured_device != dev) {
-            HYP_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(attn_kernel<D>),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-            configured_device = dev;
-        }
-    }
-    const uint32_t tiles = (p.L * p.G + kRowsPerTile - 1u) / kRowsPerTile;
-    hipLaunchKernelGGL(attn_kernel<D>, dim3(tiles, p.KVH, p.splits), dim3(kAttnThreads), lds, stream, p);
-    HYP_HIP_CHECK(hipGetLastError());
-}
-
 }  // namespace
 
 namespace {
 
-// The chunk form at most one workgroup per compute unit (a prefill chunk of up to about
-// 1024 tokens on the 12B's layers): one wave per SIMD leaves every LDS and MFMA dependency
-// exposed and the causal tiles' lengths run 1 .. L / 32 blocks. Two key splits give two
-// resident workgroups per compute unit and halve the longest tile; attn_combine_kernel
-// merges them (measured below).
-bool chunk_split_pays(uint32_t L, uint32_t n_heads, uint32_t n_kv_heads, uint32_t keys) {
-    const uint32_t G = n_heads / n_kv_heads;
-    const uint64_t tiles = (static_cast<uint64_t>(L) * G + kRowsPerTile - 1u) / kRowsPerTile * n_kv_heads;
-    return tiles <= device_compute_units() && keys >= 8u * kKeyBlock;
+// Rows of fp32 partials (m, l and head_dim values each) a split workspace holds: 64 splits of
+// the decode form's rows, or one row tile per compute unit of the chunk form (256 on MI355X; a
+// plan needs no device).
+size_t workspace_rows(uint32_t n_kv_heads) {
+    constexpr size_t kDecodeRows = 64, kPlanComputeUnits = 256;
+    return std::max(kAttnMaxSplits * kDecodeRows * n_kv_heads, kPlanComputeUnits * kChunkRows);
 }
 
-size_t chunk_split_bytes(uint32_t L, uint32_t n_heads, uint32_t head_dim) {
-    return 2u * static_cast<size_t>(L) * n_heads * (static_cast<size_t>(head_dim) * 4u + 8u);
+size_t row_bytes(uint32_t head_dim) { return static_cast<size_t>(head_dim) * 4u + 8u; }
+
+// Key splits of the chunk form: as many as the idle compute units take (one workgroup each at
+// head_dim 512, two below), with at least 4 key blocks in each (below that the merge costs
+// more than the walk) and within the workspace. Measured unsplit and by this rule: global
+// (head_dim 512, one kv head) 203 tokens behind 3000 203 -> 57 us, 64 behind 4000 251 -> 56,
+// 1000 behind 3000 250 -> 166; sliding (256, 8 kv heads) 203 behind 700 39 -> 29, 1000
+// behind 700 50 -> 43; half as many splits as the rule gives 73-81 us on the first two.
+uint32_t chunk_splits(uint32_t L, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t keys) {
+    const uint32_t G = n_heads / n_kv_heads;
+    const uint64_t tiles = (static_cast<uint64_t>(L) * G + kChunkRows - 1u) / kChunkRows * n_kv_heads;
+    const uint64_t slots = static_cast<uint64_t>(device_compute_units()) * (head_dim >= 512u ? 1u : 2u);
+    const uint64_t blocks = (keys + kKeyBlock - 1u) / kKeyBlock;
+    const uint64_t fit = workspace_rows(n_kv_heads) / (static_cast<uint64_t>(L) * n_heads);
+    const uint64_t s = std::min({slots / tiles, blocks / 4u, fit, static_cast<uint64_t>(kAttnMaxSplits)});
+    return static_cast<uint32_t>(std::max<uint64_t>(s, 1u));
 }
 
 }  // namespace
 
-size_t attention_chunk_workspace_bytes(uint32_t max_L, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim) {
-    // The longest chunk that still splits (its tiles fit the compute units), within max_L,
-    // for MI355X's 256 compute units (a plan needs no device; on a larger part the chunks
-    // this does not cover run unsplit).
-    constexpr uint64_t kPlanComputeUnits = 256;
-    const uint32_t G = n_heads / n_kv_heads;
-    const uint64_t fit = static_cast<uint64_t>(kRowsPerTile) * (kPlanComputeUnits / n_kv_heads) / G;
-    const uint32_t L = static_cast<uint32_t>(std::min<uint64_t>(max_L, fit));
-    return L > kRowsPerTile / G ? chunk_split_bytes(L, n_heads, head_dim) : 0u;
-}
-
 size_t attention_workspace_bytes(uint32_t n_kv_heads, uint32_t head_dim) {
-    // Split partials for decode: at most kAttnMaxSplits splits of one row tile per kv head.
-    const size_t rows = static_cast<size_t>(kRowsPerTile) * n_kv_heads;
-    return kAttnMaxSplits * rows * (static_cast<size_t>(head_dim) * 4u + 8u);
+    return workspace_rows(n_kv_heads) * row_bytes(head_dim);
 }
 
 void launch_kv_write(const uint16_t* k, const uint16_t* v, uint16_t* ck, uint16_t* cv, uint32_t n, uint32_t pos0,
@@ -993,16 +701,9 @@ uint32_t decode_splits(uint32_t n_kv_heads, uint32_t keys) {
     return std::max(1u, std::min(kAttnMaxSplits, (keys + kKeyBlock - 1u) / kKeyBlock));
 }
 
-uint32_t attention_splits(uint32_t L, uint32_t n_heads, uint32_t n_kv_heads, uint32_t keys) {
+uint32_t attention_splits(uint32_t L, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t keys) {
     if (static_cast<uint64_t>(L) * (n_heads / n_kv_heads) <= 16u) return decode_splits(n_kv_heads, keys);
-    // One row tile per kv head (decode): split the keys so the grid covers the compute
-    // units, at least 64 keys per split.
-    const uint32_t G = n_heads / n_kv_heads;
-    if (static_cast<uint64_t>(L) * G > kRowsPerTile) return chunk_split_pays(L, n_heads, n_kv_heads, keys) ? 2u : 1u;
-    const uint32_t cus = device_compute_units();
-    uint32_t s = 1u;
-    while (s < kAttnMaxSplits && n_kv_heads * s * 2u <= cus && keys >= 64u * (s * 2u)) s *= 2u;
-    return s;
+    return chunk_splits(L, n_heads, n_kv_heads, head_dim, keys);
 }
 
 void launch_attention(const AttnArgs& a, hipStream_t stream) {
@@ -1023,37 +724,28 @@ void launch_attention(const AttnArgs& a, hipStream_t stream) {
     p.window = a.window;
     const uint32_t T = a.prefix_len + a.L;
     p.pos = a.pos;
+    const bool decode = static_cast<uint64_t>(a.L) * p.G <= 16u;
     if (a.pos != nullptr) {
         // A grid fixed for every position the captured launch will see (the kernel
         // derives its key ranges from *pos; splits past the keys write empty partials).
         p.splits = std::max(1u, std::min(a.fixed_splits, kAttnMaxSplits));
         p.keys_per_split = kKeyBlock;
     } else {
-        p.splits = attention_splits(a.L, a.n_heads, a.n_kv_heads, T);
-        const bool chunk = static_cast<uint64_t>(a.L) * p.G > kRowsPerTile;
-        // The chunk form splits into a workspace that holds it.
-        if (chunk && p.splits > 1u &&
-            (a.workspace == nullptr || a.workspace_bytes < chunk_split_bytes(a.L, a.n_heads, a.head_dim)))
-            p.splits = 1u;
+        // (a window shows a row tile at most its own tokens' keys and a window before them)
+        const uint32_t tile_tokens = (kChunkRows + p.G - 1u) / p.G;
+        const uint32_t seen = decode || a.window == 0u ? T : std::min<uint64_t>(T, uint64_t{a.window} + tile_tokens);
+        p.splits = attention_splits(a.L, a.n_heads, a.n_kv_heads, a.head_dim, seen);
         p.keys_per_split = ((T + p.splits - 1u) / p.splits + kKeyBlock - 1u) / kKeyBlock * kKeyBlock;
-        p.splits = std::max(1u, (T + p.keys_per_split - 1u) / p.keys_per_split);   // no empty split
+        if (decode) p.splits = std::max(1u, (T + p.keys_per_split - 1u) / p.keys_per_split);   // no empty split
     }
-    if (p.splits > 1u && static_cast<uint64_t>(a.L) * p.G > kRowsPerTile) {
-        // chunk form: checked above
+    if (p.splits > 1u) {
         const size_t rows = static_cast<size_t>(a.L) * a.n_heads;
-        p.part_o = static_cast<float*>(a.workspace);
-        p.part_ml = reinterpret_cast<float*>(static_cast<uint8_t*>(a.workspace) +
-                                             static_cast<size_t>(p.splits) * rows * a.head_dim * 4u);
-    } else if (p.splits > 1u) {
-        HYP_REQUIRE(a.workspace != nullptr &&
-                        a.workspace_bytes >= attention_workspace_bytes(a.n_kv_heads, a.head_dim),
+        HYP_REQUIRE(a.workspace != nullptr && a.workspace_bytes >= p.splits * rows * row_bytes(a.head_dim),
                     HYP_STATUS_INTERNAL, "attention: split workspace too small");
-        const size_t rows = static_cast<size_t>(a.L) * a.n_heads;
         p.part_o = static_cast<float*>(a.workspace);
         p.part_ml = reinterpret_cast<float*>(static_cast<uint8_t*>(a.workspace) +
                                              static_cast<size_t>(p.splits) * rows * a.head_dim * 4u);
     }
-    const bool decode = static_cast<uint64_t>(a.L) * p.G <= 16u;
     const bool prep = a.prep != nullptr;
     if (prep) {
         const AttnPrepareArgs& pa = *a.prep;
@@ -1072,15 +764,19 @@ void launch_attention(const AttnArgs& a, hipStream_t stream) {
         p.cv_out = pa.cache_v;
         p.eps = pa.eps;
     }
-    switch (a.head_dim) {
-        case 64: decode ? launch_decode_d<64>(p, prep, stream) : launch_attn_d<64>(p, stream); break;
-        case 128: decode ? launch_decode_d<128>(p, prep, stream) : launch_attn_d<128>(p, stream); break;
-        case 256: decode ? launch_decode_d<256>(p, prep, stream) : launch_attn_d<256>(p, stream); break;
-        case 512: decode ? launch_decode_d<512>(p, prep, stream) : launch_attn_d<512>(p, stream); break;
-        default: throw NativeError(HYP_STATUS_UNSUPPORTED, "attention: head_dim must be 64, 128, 256 or 512");
+    if (!decode) {
+        launch_attn_chunk(p, a.head_dim, stream);
+    } else {
+        switch (a.head_dim) {
+            case 64: launch_decode_d<64>(p, prep, stream); break;
+            case 128: launch_decode_d<128>(p, prep, stream); break;
+            case 256: launch_decode_d<256>(p, prep, stream); break;
+            case 512: launch_decode_d<512>(p, prep, stream); break;
+            default: throw NativeError(HYP_STATUS_UNSUPPORTED, "attention: head_dim must be 64, 128, 256 or 512");
+        }
     }
-    if (p.splits > 1u && static_cast<uint64_t>(a.L) * p.G > kRowsPerTile) {
-        // chunk form: many rows, two splits; a thread per 8 dims of a row
+    if (p.splits > 1u && !decode) {
+        // chunk form: many rows, few splits; a thread per 8 dims of a row
         const uint64_t threads = static_cast<uint64_t>(a.L) * a.n_heads * (a.head_dim / 8u);
         const uint64_t blocks = (threads + kAttnThreads - 1u) / kAttnThreads;
         HYP_REQUIRE(blocks <= 0x7fffffffull, HYP_STATUS_INVALID_ARGUMENT, "attention: too many rows to merge");

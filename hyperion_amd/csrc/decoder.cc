@@ -162,14 +162,10 @@ uint64_t rope_table_bytes(const Geometry& g, uint32_t D) {
     return bytes > kRopeTableMaxBytes ? 0u : bytes;
 }
 
-// The attention split workspace: decode splits, and the chunk form's two key splits up to
-// one prefill chunk, for both layer kinds.
+// The attention split workspace of both layer kinds.
 uint64_t attention_ws_bytes(const Geometry& g) {
-    const uint32_t chunk = std::min(kChunkTokens, g.max_positions);
-    return std::max({hip::attention_workspace_bytes(g.kv_heads_local, g.head_dim_local),
-                     hip::attention_workspace_bytes(g.kv_heads_global, g.head_dim_global),
-                     hip::attention_chunk_workspace_bytes(chunk, g.heads, g.kv_heads_local, g.head_dim_local),
-                     hip::attention_chunk_workspace_bytes(chunk, g.heads, g.kv_heads_global, g.head_dim_global)});
+    return std::max(hip::attention_workspace_bytes(g.kv_heads_local, g.head_dim_local),
+                    hip::attention_workspace_bytes(g.kv_heads_global, g.head_dim_global));
 }
 
 }  // namespace
@@ -486,7 +482,7 @@ void Decoder::forward_chunk(DecoderState& st, const uint32_t* d_ids, uint32_t L,
             // Splits sized for the longest key range the replays can see.
             const uint32_t max_keys = sliding ? std::min(g.window, g.max_positions) + L : g.max_positions;
             aa.pos = d_pos;
-            aa.fixed_splits = hip::attention_splits(L, g.heads, kvh, max_keys);
+            aa.fixed_splits = hip::attention_splits(L, g.heads, kvh, D, max_keys);
         }
         if (fold_prepare) aa.prep = &pa;
         hip::launch_attention(aa, s);

@@ -87,6 +87,56 @@ def test_attention_matches_oracle(stream, L, H, KVH, D, cap, offset, prefix, win
     cache.close()
 
 
+CHUNK_CASES = [
+    # L, H, KVH, D, cap, offset, prefix, window, chunk in the cache
+    (17, 4, 4, 64, 64, 5, 5, 0, True),            # one row per token, one more than the decode form takes
+    (33, 4, 1, 64, 64, 20, 20, 24, True),         # 132 rows: 4 past a row tile; window edges in a block
+    (32, 8, 2, 128, 40, 101, 8, 8, True),         # 128 rows exactly; the ring wraps inside a block
+    (31, 8, 2, 128, 40, 77, 9, 10, False),        # chunk beside a wrapped prefix
+    (129, 2, 2, 256, 300, 1000, 171, 172, True),  # one row past a tile, prefix + chunk fill the ring
+    (5, 16, 1, 512, 700, 650, 650, 0, True),      # many key splits of one partial tile
+    (70, 16, 1, 512, 2200, 2100, 2100, 0, True),  # splits whose causal end is inside the last block
+    (64, 16, 1, 512, 16, 33, 16, 0, False),       # a ring of half a key block
+]
+
+
+@pytest.mark.parametrize("L,H,KVH,D,cap,offset,prefix,window,cached", CHUNK_CASES)
+def test_chunk_kernel_edges(stream, L, H, KVH, D, cap, offset, prefix, window, cached):
+    """The chunk kernel at the edges of its row tiles, key blocks, splits and rings. One cached
+    K row is NaN: its scores count as masked. Slots no position maps to hold NaN and must not
+    reach a result. Bar as above."""
+    say(f"chunk attention L={L} KVH={KVH} D={D} cap={cap} offset={offset} prefix={prefix} window={window}")
+    rng = np.random.default_rng(L * 31 + D + cap)
+    b = lambda scale, *shape: syn.bf16_bits((rng.standard_normal(shape) * scale).astype(np.float32))  # noqa: E731
+    nan = np.uint16(0x7FC0)
+    q, k, v = b(D ** -0.5 * 2.0, L, H, D), b(1.0, L, KVH, D), b(1.0, L, KVH, D)
+    ck, cv = np.full((cap, KVH, D), nan), np.full((cap, KVH, D), nan)
+    for p in range(offset - prefix, offset):
+        ck[p % cap], cv[p % cap] = b(1.0, KVH, D), b(1.0, KVH, D)
+    dead = prefix // 2                      # index of the NaN key, in the oracle a very negative one
+    ckr, cvr = ck.copy(), cv.copy()
+    ckr[ck == nan], cvr[cv == nan] = 0, 0
+    slot = (offset - prefix + dead) % cap
+    ck[slot] = nan
+    q[:, :, 0] = syn.bf16_bits(-np.maximum(np.abs(syn.bf16_to_f32(q[:, :, 0])), 0.01).astype(np.float32))
+    ckr[slot] = 0
+    ckr[slot, :, 0] = syn.bf16_bits(np.full((KVH,), 1e6, np.float32))   # score <= -1e4: weight 0
+    ref = O.attention_f64(q, k, v, ckr, cvr, offset, prefix, window)
+    cache = hy.KvCache(cap, KVH, D)
+    if cached:
+        for t in range(L):
+            ck[(offset + t) % cap], cv[(offset + t) % cap] = k[t], v[t]
+    _fill_cache(cache, ck, cv, stream)
+    qd, kd, vd = dev(q, stream), dev(k, stream), dev(v, stream)
+    out = hy.DeviceArray((L, H, D), np.uint16)
+    hy.call("hyp_attention", qd.ptr, None if cached else kd.ptr, None if cached else vd.ptr, L, H, cache.handle, offset,
+            prefix, window, out.ptr, stream.handle)
+    _check(out.to_host(stream), ref, np.concatenate([v.reshape(-1), cvr.reshape(-1)]), f"L={L} D={D}")
+    for a in (qd, kd, vd, out):
+        a.close()
+    cache.close()
+
+
 def test_kv_cache_write_slots_and_ring_overwrite(stream):
     """Tokens land in slot p % capacity; a write longer than the ring keeps its last
     `capacity` tokens; attention over the written prefix equals attention over the same
