@@ -802,6 +802,134 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2))) 
     }
 }
 
+// ---- few rows: a wave per (column tiles, k range) ----------------------------------------
+//
+// Up to a few dozen rows the weight stream and X's reads bound a call, not the matrix
+// products, and the tile kernels use 16 rows of their 128, wait for their loads at a barrier
+// per step, and leave most compute units idle (down: 30 column tiles, 4 splits). Here, as in
+// the decode kernel, a wave takes NT 16-column tiles (DUAL: gate and up tiles in turn) and a
+// contiguous range of their group pairs, with its weights and its X rows two pairs ahead in
+// registers (X from L2, straight in the A operand's layout: lane (i, kb) reads 16 bytes of row
+// i), no barrier in the loop; the `splits` waves of a tile are neighbours in a workgroup and
+// add up through LDS in wave order, so nothing is left to a second launch. Weights
+// dequantize as in the tile kernels (bf16(scale q + bias)). More than two pairs ahead or 16
+// waves per workgroup measured the same or slower (q/k/v at 16 rows 10.6 -> 11.4 with 4 pairs).
+constexpr uint32_t kFewRows = 64;   // at most
+constexpr uint32_t kFewWaves = 8;
+
+template <int MT, int NT, bool DUAL>
+__global__ __launch_bounds__(64 * kFewWaves) void q4_gemm_few_kernel(GemmParams p) {
+    constexpr int DEPTH = 2;
+    static_assert(!DUAL || NT % 2 == 0, "a dual launch pairs gate and up tiles");
+    constexpr int kOut = DUAL ? NT / 2 : NT;   // output column tiles per wave
+    extern __shared__ __attribute__((aligned(16))) uint8_t xs[];   // [kFewWaves][MT][NT][4][64] fp32
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t splits = p.ksplit;
+    const uint32_t per_wg = kFewWaves / splits;
+    const uint32_t sub = wave / splits;                       // tile of the workgroup
+    const uint32_t z = wave - sub * splits;                   // k range of the tile
+    const uint32_t tn = min(blockIdx.x * per_wg + sub, p.tiles_n - 1u);
+    const SegView sv = view_of<DUAL>(p, tn);
+    const uint32_t k = p.k;
+    const uint32_t p0 = p.pairs * z / splits;
+    const uint32_t p1 = p.pairs * (z + 1u) / splits;          // not empty: splits <= pairs
+
+    const uint32_t i = lane & 15u;
+    const uint32_t kb = lane >> 4;
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(p.x), static_cast<short>(0), static_cast<int>(p.m * k * 2u), 0x00020000);
+    const WeightRsrc wr = weight_rsrc<DUAL>(p, sv);
+    uint32_t c_off[NT];
+    uint32_t s_off[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        // (DUAL: even nt of the gate, odd of up; tiles past the last repeat it, never stored)
+        const uint32_t t16 = min(sv.tn * kOut + (DUAL ? nt / 2 : nt), sv.row_tiles - 1u);
+        c_off[nt] = (t16 * p.pairs * 64u + lane) * 16u;
+        s_off[nt] = (t16 * p.pairs * 16u + i) * 8u;
+    }
+    // Rows past m, and the second group of the last pair of an odd group count, load zeros (an
+    // offset past the resource).
+    uint32_t xoff[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const uint32_t row = 16u * mt + i;
+        xoff[mt] = row < p.m ? row * k * 2u + kb * 32u : 0x80000000u;
+    }
+    const uint32_t last_full = k / kPairK;   // pairs below it hold two groups
+
+    BRaw<NT> raw[DEPTH];
+    bf16x8_t a[DEPTH][MT][4];
+    const auto load = [&](uint32_t pair, BRaw<NT>& r, bf16x8_t (&av)[MT][4]) {
+        const uint32_t pn = min(pair, p1 - 1u);
+        load_b<NT>(wr, c_off, s_off, pn, r);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int st = 0; st < 4; ++st) {
+                const uint32_t off = st >= 2 && pn >= last_full ? 0x80000000u : xoff[mt] + (st / 2) * 128u + (st % 2) * 16u;
+                av[mt][st] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                              xr, static_cast<int>(off), static_cast<int>(pn * 256u), 0));
+            }
+    };
+    f32x4_t acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) load(p0 + d, raw[d], a[d]);
+    const auto step = [&](auto sc, const BRaw<NT>& r, const bf16x8_t (&av)[MT][4]) {
+        constexpr int S = decltype(sc)::value;
+        bf16x8_t b[NT];
+        dequant_step<NT, S>(r, b);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+                acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[mt][S], b[nt], acc[mt][nt], 0, 0, 0);
+    };
+    for (uint32_t pair = p0; pair < p1; pair += DEPTH) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            if (pair + d < p1) {
+                static_for([&](auto sc) { step(sc, raw[d], a[d]); }, std::make_integer_sequence<int, 4>{});
+                if (pair + d + DEPTH < p1) load(pair + d + DEPTH, raw[d], a[d]);
+            }
+        }
+    }
+
+    // acc[mt][nt][r] is (row 16 mt + 4 kb + r, column i) of the tile.
+    float* part = reinterpret_cast<float*>(xs);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[(((wave * MT + mt) * NT + nt) * 4u + r) * 64u + lane] = acc[mt][nt][r];
+    __syncthreads();
+    constexpr uint32_t kOuts = MT * kOut * 256u;   // outputs of a wave's tiles: (mt, tile, r, lane)
+    for (uint32_t e = threadIdx.x; e < per_wg * kOuts; e += 64u * kFewWaves) {
+        const uint32_t t = e / kOuts;
+        const uint32_t o = e - t * kOuts;
+        const uint32_t l = o & 63u;
+        const uint32_t r = (o >> 6) & 3u;
+        const uint32_t ot = (o >> 8) % kOut;
+        const uint32_t mt = (o >> 8) / kOut;
+        if (blockIdx.x * per_wg + t >= p.tiles_n) break;
+        const SegView ov = view_of<DUAL>(p, blockIdx.x * per_wg + t);
+        const uint32_t row = 16u * mt + 4u * (l >> 4) + r;
+        const uint32_t col = (ov.tn * kOut + ot) * 16u + (l & 15u);
+        if (row >= p.m || col >= ov.n) continue;
+        float sum[2] = {0.0f, 0.0f};
+#pragma unroll
+        for (int d = 0; d < (DUAL ? 2 : 1); ++d)
+            for (uint32_t w = 0; w < splits; ++w)
+                sum[d] += part[((((t * splits + w) * MT + mt) * NT + (DUAL ? 2u * ot + d : ot)) * 4u + r) * 64u + l];
+        ov.y[static_cast<size_t>(row) * ov.n + col] = DUAL ? gated_bits(sum[0], sum[1]) : f32_to_bf16_bits(sum[0]);
+    }
+}
 
 // The same with 8 consecutive workspace columns per thread (two 16-byte loads per split,
 // one 16-byte store), for grids where every segment's width and first column are
@@ -947,6 +1075,69 @@ void launch_g(GemmParams p, hipStream_t stream) {
     const uint32_t tiles_m = (p.m + 16u * MT - 1u) / (16u * MT);
     p.tiles_total = p.tiles_n * tiles_m;
     hipLaunchKernelGGL(kernel, dim3(p.tiles_total * p.ksplit), dim3(64 * W), lds, stream, p);
+}
+
+template <int MT, int NT, bool DUAL>
+void launch_few_t(GemmParams p, hipStream_t stream) {
+    constexpr size_t lds = size_t{kFewWaves} * MT * NT * 1024u;
+    static_assert(lds <= 65536u, "few-row GEMM LDS");
+    retile(p, 16u * (DUAL ? NT / 2 : NT));
+    const uint32_t per_wg = kFewWaves / p.ksplit;
+    const uint32_t grid = (p.tiles_n + per_wg - 1u) / per_wg;
+    hipLaunchKernelGGL((q4_gemm_few_kernel<MT, NT, DUAL>), dim3(grid), dim3(64 * kFewWaves), lds, stream, p);
+    HYP_HIP_CHECK(hipGetLastError());
+}
+
+template <int MT>
+void launch_few_m(const GemmParams& p, uint32_t nt, hipStream_t stream) {
+    if (p.dual != 0u) {
+        if constexpr (MT <= 2) {
+            if (nt == 4u) return launch_few_t<MT, 4, true>(p, stream);
+        }
+        return launch_few_t<MT, 2, true>(p, stream);
+    }
+    if constexpr (MT <= 2) {
+        if (nt == 4u) return launch_few_t<MT, 4, false>(p, stream);
+    }
+    nt >= 2u ? launch_few_t<MT, 2, false>(p, stream) : launch_few_t<MT, 1, false>(p, stream);
+}
+
+// Whether the few-row kernel takes the call. Its time grows with rows x column tiles (each
+// wave reads its rows of X from L2, about 12 TB/s over the chip), the tile kernels' hardly
+// below 128 rows. Measured, tile kernels against it (us, weights alternating): gate + up
+// [2 x 15360, 3840] 38.8 -> 20.8 at 16 rows, 37.4 -> 27.5 at 32, but 37.5 -> 42.5 at 33; down
+// [3840, 15360] 56.4 -> 11.9 at 5, 18.8 at 16, 31.4 at 32, 45.6 at 48, 58.0 -> 58.6 at 64; q/k/v
+// [8192, 3840] 25.3 -> 8.8 at 16, 27.1 -> 19.5 at 64; o [3840, 4096] 23.5 -> 7.2 at 16, 25.6 ->
+// 18.8 at 64; [15360, 3840] 27.1 -> 16.9 at 32, 28.9 -> 35.2 at 64; [262144, 3840] 323 -> 190 at
+// 32. So: always up to 32 rows, to 64 where the column tiles are at most two per compute unit.
+bool few_rows(const GemmParams& p) {
+    uint64_t tiles = 0;
+    for (uint32_t i = 0; i < p.nseg; ++i) tiles += p.seg[i].row_tiles;
+    return p.m <= 32u || (p.m <= kFewRows && tiles <= 2u * device_compute_units());
+}
+
+void launch_few(GemmParams p, hipStream_t stream) {
+    // As many column tiles per wave (they share its X reads) as leave 7 waves per compute unit
+    // with every tile's pairs over 8 waves, then the fewest waves per tile that still do; from
+    // 33 rows on at most 2 (registers, and the LDS of the sums). At 16 rows (us): [15360, 3840]
+    // 18.7, 13.2 and 12.0 with 1, 2 and 4 tiles per wave, q/k/v [8192, 3840] 10.9, 8.5 and 11.4,
+    // down [3840, 15360] 19.0, 21.5 and 30.1.
+    const uint64_t cus = device_compute_units();
+    uint64_t tiles = 0;
+    for (uint32_t i = 0; i < p.nseg; ++i) tiles += p.seg[i].row_tiles;
+    const uint32_t nt_max = p.m <= 32u ? 4u : 2u;
+    uint32_t nt = p.dual != 0u ? 2u : 1u;
+    while (nt < nt_max && tiles / (2u * nt) * kFewWaves >= 7u * cus) nt *= 2u;
+    uint32_t s = 1u;
+    while (s < kFewWaves && tiles / nt * s < 7u * cus && 2u * s <= p.pairs) s *= 2u;
+    p.ksplit = s;
+    switch ((p.m + 15u) / 16u) {
+        case 1: launch_few_m<1>(p, nt, stream); break;
+        case 2: launch_few_m<2>(p, nt, stream); break;
+        case 3: launch_few_m<3>(p, nt, stream); break;
+        case 4: launch_few_m<4>(p, nt, stream); break;
+        default: throw NativeError(HYP_STATUS_INTERNAL, "gemm: too many rows for the few-row kernel");
+    }
 }
 
 // Parameters of a grouped launch; tiles_total is set by the launcher of the chosen kernel.
@@ -1147,6 +1338,7 @@ float* noalloc_scratch() {
 void launch_q4_gemm_group(const Q4Matrix* const* ws, uint16_t* const* ys, uint32_t count, const uint16_t* x,
                           uint32_t m, hipStream_t stream) {
     GemmParams p = group_params(ws, ys, count, x, m);
+    if (few_rows(p)) return launch_few(p, stream);
     const GemmChoice c = choose_gemm(p);
     launch_split(p, c.kernel, c.ksplit, stream);
 }
@@ -1159,6 +1351,7 @@ void launch_q4_gemm_gate_up(const Q4Matrix& gate, const Q4Matrix& up, const uint
     GemmParams p = group_params(ws, ys, 2u, x, m);
     const GemmChoice c = choose_gemm(p);   // the kernel and split of the grouped gate/up launch
     p.dual = 1u;
+    if (few_rows(p)) return launch_few(p, stream);
     launch_split(p, c.kernel, c.ksplit, stream);
 }
 
@@ -1172,7 +1365,9 @@ void launch_q4_gemm_noalloc(const Q4Matrix& w, const uint16_t* x, uint32_t m, ui
     const Q4Matrix* ws[1] = {&w};
     uint16_t* ys[1] = {y};
     GemmParams p = group_params(ws, ys, 1u, x, m);
-    const GemmChoice c = choose_gemm(p);   // the same kernel and split as launch_q4_gemm
+    // The same kernel and split as launch_q4_gemm.
+    if (few_rows(p)) return launch_few(p, stream);
+    const GemmChoice c = choose_gemm(p);
     SplitWorkspace wsp;
     wsp.fixed = noalloc_scratch();
     wsp.fixed_bytes = kNoAllocScratchBytes;

@@ -439,6 +439,45 @@ def test_gemm_split_k_grouped_and_exact(stream):
     np.testing.assert_array_equal(y2, syn.bf16_bits(exact.astype(np.float32)))
 
 
+FEW_CASES = [
+    # m, widths, k: row tiles of 16 with 1..16 rows in the last, 1 to 8 waves per column tile
+    (5, (33,), 64),                 # one pair, its second group past k
+    (16, (40, 24, 1000), 192),      # two pairs; segments of part-empty column tiles
+    (17, (1000,), 4160),            # a second row tile of one row; odd group count
+    (32, (520, 33), 1024),
+    (32, (15360,), 448),            # four column tiles per wave
+    (31, (8200,), 320),             # two, the last wave's second past the end
+    (33, (2048, 16), 1088),
+    (48, (4096, 2048, 2041), 256),  # 513 column tiles: the tile kernels again from 33 rows on
+    (64, (3840,), 704),
+]
+
+
+@pytest.mark.parametrize("m,ns,k", FEW_CASES)
+def test_gemm_few_rows_exact(stream, m, ns, k):
+    """The few-row kernel at the edges of its tiles and splits: integer inputs, whose sums are
+    exact in fp32 in any order, so every output equals the exact product rounded once; X rows past m and groups past k must
+    not contribute (the row after the last is NaN)."""
+    say(f"few rows m={m} ns={ns} k={k}")
+    rng = np.random.default_rng(m * 100 + k)
+    x = rng.integers(-1, 2, size=(m + 1, k)).astype(np.float32)
+    x[m] = np.nan
+    xd = dev(syn.bf16_bits(x), stream)
+    qws, ys, exact = [], [], []
+    for n in ns:
+        codes = rng.integers(0, 16, size=(n, k)).astype(np.uint8)
+        s = syn.bf16_bits(np.full((n, k // 64), 2.0**-7, np.float32))
+        b = syn.bf16_bits(np.full((n, k // 64), -(2.0**-4), np.float32))
+        qws.append(hy.QWeight.from_host(syn.pack_codes(codes), s, b))
+        ys.append(hy.DeviceArray((m, n), np.uint16))
+        exact.append((x[:m].astype(np.int64) @ (codes.astype(np.int64) - 8).T) * 2.0**-7)
+    hy.qmatmul_group(qws, xd, m, ys, stream)
+    for n, y, e in zip(ns, ys, exact):
+        np.testing.assert_array_equal(y.to_host(stream), syn.bf16_bits(e.astype(np.float32)), err_msg=f"n={n}")
+    for a in (*qws, *ys, xd):
+        a.close()
+
+
 @pytest.mark.parametrize("n,k", [(8200, 192), (8195, 320), (8200, 3840)])
 def test_gemm_group_step_tiles(stream, n, k):
     """Grids of >= 0.9 workgroups per CU in 256 x 256 tiles select the 256-row group-step kernel: ragged m
