@@ -59,6 +59,11 @@ __device__ __forceinline__ const uint16_t* key_row(const AttnParams& p, const ui
     return chunk + (static_cast<size_t>(j - p.prefix) * p.KVH + hk) * D;
 }
 
+// Splits of the decode form that hold keys (of the p.splits of its grid).
+__device__ __forceinline__ uint32_t used_splits(const AttnParams& p) {
+    return min(p.splits, (p.prefix + p.L + p.keys_per_split - 1u) / p.keys_per_split);
+}
+
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef short short8_t __attribute__((ext_vector_type(8)));
 
@@ -177,7 +182,7 @@ __global__ __launch_bounds__(DecodeLds<D>::kWaves * 64u) void attn_decode_kernel
     // and their branches then stay scalar rather than masking lanes around the loads.
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t split = blockIdx.x * Lds::kWaves + wave;
-    if (split >= p.splits) return;   // no workgroup barrier below: waves are independent
+    if (split >= used_splits(p)) return;   // no workgroup barrier below: waves are independent
     const uint32_t hk = blockIdx.y;
     const uint32_t j16 = lane & 15u;
     const uint32_t kb = lane >> 4;
@@ -368,54 +373,49 @@ __global__ __launch_bounds__(DecodeLds<D>::kWaves * 64u) void attn_decode_kernel
     }
 
     // Per 16-key column tile c: K rows into the B operands, V rows (coalesced, lane cidx takes
-    // chunk cidx % (D/8) of key cidx / (D/8)) into registers, every load of the tile issued
-    // before its first use; with D <= 256 both tiles' loads are issued together.
+    // chunk cidx % (D/8) of key cidx / (D/8)) into registers, every load of the block's two
+    // tiles issued before the first use (at head_dim 512 256 registers of them, of the 512 a
+    // wave has where LDS lets one wave on a SIMD: 262000 keys 206 -> 188 us).
     constexpr uint32_t kChunks = D / 8u;
     constexpr uint32_t kVPer = 16u * kChunks / 64u;   // V chunks per lane per 16-key tile
-    constexpr uint32_t kTilesUpFront = D <= 256u ? 2u : 1u;
     for (uint32_t jb = j_begin; jb < j_end; jb += kKeyBlock) {
         const uint32_t nk = min(kKeyBlock, j_end - jb);
         f32x4_t sc[2] = {f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}};
+        uint4 kr[2u][kSteps];
+        uint4 vr[2u][kVPer];
 #pragma unroll
-        for (uint32_t c0 = 0; c0 < 2u; c0 += kTilesUpFront) {
-            uint4 kr[kTilesUpFront][kSteps];
-            uint4 vr[kTilesUpFront][kVPer];
+        for (uint32_t c = 0; c < 2u; ++c) {
+            const uint32_t key = 16u * c + j16;
+            const uint16_t* row = key < nk ? key_row(p, p.k, p.ck, jb + key, hk, D) + kb * 8u : nullptr;
 #pragma unroll
-            for (uint32_t u = 0; u < kTilesUpFront; ++u) {
-                const uint32_t c = c0 + u;
-                const uint32_t key = 16u * c + j16;
-                const uint16_t* row = key < nk ? key_row(p, p.k, p.ck, jb + key, hk, D) + kb * 8u : nullptr;
-#pragma unroll
-                for (uint32_t st = 0; st < kSteps; ++st) {
-                    kr[u][st] = row != nullptr ? *reinterpret_cast<const uint4*>(row + st * 32u)
-                                               : make_uint4(0u, 0u, 0u, 0u);
-                }
-#pragma unroll
-                for (uint32_t it = 0; it < kVPer; ++it) {
-                    const uint32_t cidx = lane + 64u * it;
-                    const uint32_t r = 16u * c + cidx / kChunks;
-                    const uint32_t ch = cidx % kChunks;
-                    vr[u][it] = r < nk ? *reinterpret_cast<const uint4*>(key_row(p, p.v, p.cv, jb + r, hk, D) + ch * 8u)
-                                       : make_uint4(0u, 0u, 0u, 0u);
-                }
+            for (uint32_t st = 0; st < kSteps; ++st) {
+                kr[c][st] = row != nullptr ? *reinterpret_cast<const uint4*>(row + st * 32u)
+                                           : make_uint4(0u, 0u, 0u, 0u);
             }
 #pragma unroll
-            for (uint32_t u = 0; u < kTilesUpFront; ++u) {
-                const uint32_t c = c0 + u;
-                // V rows into LDS as loaded.
+            for (uint32_t it = 0; it < kVPer; ++it) {
+                const uint32_t cidx = lane + 64u * it;
+                const uint32_t r = 16u * c + cidx / kChunks;
+                const uint32_t ch = cidx % kChunks;
+                vr[c][it] = r < nk ? *reinterpret_cast<const uint4*>(key_row(p, p.v, p.cv, jb + r, hk, D) + ch * 8u)
+                                   : make_uint4(0u, 0u, 0u, 0u);
+            }
+        }
 #pragma unroll
-                for (uint32_t it = 0; it < kVPer; ++it) {
-                    const uint32_t cidx = lane + 64u * it;
-                    const uint32_t r = 16u * c + cidx / kChunks;
-                    const uint32_t ch = cidx % kChunks;
-                    *reinterpret_cast<uint4*>(my + Lds::kV + r * Lds::kVRow + ch * 16u) = vr[u][it];
-                }
-                // S for this tile's 16 keys.
+        for (uint32_t c = 0; c < 2u; ++c) {
+            // V rows into LDS as loaded.
 #pragma unroll
-                for (uint32_t st = 0; st < kSteps; ++st) {
-                    sc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa[st], __builtin_bit_cast(bf16x8_t, kr[u][st]),
-                                                                    sc[c], 0, 0, 0);
-                }
+            for (uint32_t it = 0; it < kVPer; ++it) {
+                const uint32_t cidx = lane + 64u * it;
+                const uint32_t r = 16u * c + cidx / kChunks;
+                const uint32_t ch = cidx % kChunks;
+                *reinterpret_cast<uint4*>(my + Lds::kV + r * Lds::kVRow + ch * 16u) = vr[c][it];
+            }
+            // S for this tile's 16 keys.
+#pragma unroll
+            for (uint32_t st = 0; st < kSteps; ++st) {
+                sc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa[st], __builtin_bit_cast(bf16x8_t, kr[c][st]),
+                                                                sc[c], 0, 0, 0);
             }
         }
         // Mask, online softmax (log2 domain), P -> LDS as bf16.
@@ -485,71 +485,79 @@ __global__ __launch_bounds__(DecodeLds<D>::kWaves * 64u) void attn_decode_kernel
     }
 }
 
-// Merge the splits of each output row: weights 2^(m_s - max m), sum of l_s, divided sums.
-// One workgroup per row and 256 dims (two per row at head_dim 512: 10.8 -> 4.x us for the
-// 12B's global rows), every load issued at once: each wave reads all (m, l) (lane s holds
-// split s) and the partial rows of splits w, w + 4, ... (lane-owned dims); the four wave
-// sums meet in LDS and are added in wave order.
+// Merge the splits of each output row: weights 2^(m_s - max m), sum of l_s, divided sums. One
+// workgroup per row and 64 dims: thread t weighs split t through LDS; lane (g, c) of the 16
+// groups of 16 lanes sums splits g, g + 16, ... of dims 4c .. 4c + 3, every load issued at
+// once before the weights are known, and the 16 sums meet in LDS in order. Splits past the
+// last key are not read (the decode kernel writes nothing for them).
 template <uint32_t D>
 __global__ __launch_bounds__(kAttnThreads) void attn_combine_kernel(AttnParams p) {
-    constexpr uint32_t kWaves = kAttnThreads / 64u;
-    constexpr uint32_t kDW = D < 256u ? D : 256u;   // dims of this workgroup: [d0, d0 + kDW)
-    constexpr uint32_t kPer = kDW / 64u;
-    constexpr uint32_t kMaxPerWave = kAttnMaxSplits / kWaves;
-    __shared__ float acc[kWaves][kDW];
-    __shared__ float dens[kWaves];
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = threadIdx.x >> 6;
+    static_assert(kAttnMaxSplits <= kAttnThreads, "a thread per split");
+    constexpr uint32_t kGroups = kAttnThreads / 16u;
+    constexpr uint32_t kPer = kAttnMaxSplits / kGroups;
+    __shared__ float weight[kAttnThreads];
+    __shared__ float red[2][kAttnThreads / 64u];
+    __shared__ float4 acc[kGroups][16];
+    resolve_position(p);
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid & 63u;
+    const uint32_t splits = used_splits(p);
     const uint64_t rows = static_cast<uint64_t>(p.L) * p.H;
     const uint64_t row = blockIdx.x;
-    const uint32_t d0 = blockIdx.y * kDW;
+    const uint32_t g = tid >> 4;
+    const uint32_t d0 = blockIdx.y * 64u + (tid & 15u) * 4u;
     float ms = -__builtin_huge_valf();
     float ls = 0.0f;
-    if (lane < p.splits) {
-        ms = p.part_ml[(lane * rows + row) * 2u];
-        ls = p.part_ml[(lane * rows + row) * 2u + 1u];
+    if (tid < splits) {
+        const float2 ml = *reinterpret_cast<const float2*>(p.part_ml + (tid * rows + row) * 2u);
+        ms = ml.x;
+        ls = ml.y;
     }
-    float part[kMaxPerWave][kPer];
+    float4 part[kPer];
 #pragma unroll
-    for (uint32_t u = 0; u < kMaxPerWave; ++u) {
-        const uint32_t sp = wave + kWaves * u;
-        const float* o = p.part_o + (sp * rows + row) * D + d0 + lane * kPer;
-#pragma unroll
-        for (uint32_t e = 0; e < kPer; ++e) part[u][e] = sp < p.splits ? o[e] : 0.0f;
+    for (uint32_t u = 0; u < kPer; ++u) {
+        const uint32_t sp = g + kGroups * u;
+        part[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (sp < splits) part[u] = *reinterpret_cast<const float4*>(p.part_o + (sp * rows + row) * D + d0);
     }
-    const float mx = butterfly_max64(ms, lane);
-    const float w = ms == -__builtin_huge_valf() || mx == -__builtin_huge_valf() ? 0.0f : exp2f(ms - mx);
-    float num[kPer];
-#pragma unroll
-    for (uint32_t e = 0; e < kPer; ++e) num[e] = 0.0f;
-    float den = 0.0f;
-#pragma unroll
-    for (uint32_t u = 0; u < kMaxPerWave; ++u) {
-        const uint32_t sp = wave + kWaves * u;
-        // Split sp's weight and l from lane sp (sp is uniform: a scalar read of one lane).
-        const float ws = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), static_cast<int>(sp & 63u)));
-        const float lw = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ls), static_cast<int>(sp & 63u)));
-        if (sp >= p.splits || ws == 0.0f) continue;   // uniform: past the splits, or an empty split
-        den += ws * lw;
-#pragma unroll
-        for (uint32_t e = 0; e < kPer; ++e) num[e] += ws * part[u][e];
-    }
-#pragma unroll
-    for (uint32_t e = 0; e < kPer; ++e) acc[wave][lane * kPer + e] = num[e];
-    if (lane == 0u) dens[wave] = den;
+    float mx = butterfly_max64(ms, lane);
+    if (lane == 0u) red[0][tid >> 6] = mx;
     __syncthreads();
-    if (wave != 0u) return;
-    float dt = 0.0f;
+    mx = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+    const float w = ms == -__builtin_huge_valf() || mx == -__builtin_huge_valf() ? 0.0f : exp2f(ms - mx);
+    weight[tid] = w;
+    const float den_w = butterfly_sum<32u>(w == 0.0f ? 0.0f : w * ls, lane);
+    if (lane == 0u) red[1][tid >> 6] = den_w;
+    __syncthreads();
+    float4 num = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
-    for (uint32_t wv = 0; wv < kWaves; ++wv) dt += dens[wv];
-    uint16_t* out = p.out + row * D + d0 + lane * kPer;
-#pragma unroll
-    for (uint32_t e = 0; e < kPer; ++e) {
-        float v = 0.0f;
-#pragma unroll
-        for (uint32_t wv = 0; wv < kWaves; ++wv) v += acc[wv][lane * kPer + e];
-        out[e] = f32_to_bf16_bits(dt > 0.0f ? v / dt : 0.0f);
+    for (uint32_t u = 0; u < kPer; ++u) {
+        const uint32_t sp = g + kGroups * u;
+        const float ws = weight[sp];
+        if (sp >= splits || ws == 0.0f) continue;   // an empty split's O is not used
+        num.x += ws * part[u].x;
+        num.y += ws * part[u].y;
+        num.z += ws * part[u].z;
+        num.w += ws * part[u].w;
     }
+    acc[g][tid & 15u] = num;
+    __syncthreads();
+    if (tid >= 16u) return;
+    const float den = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (uint32_t q = 0; q < kGroups; ++q) {
+        const float4 a = acc[q][tid];
+        v.x += a.x;
+        v.y += a.y;
+        v.z += a.z;
+        v.w += a.w;
+    }
+    const bool any = den > 0.0f;
+    uint2 out;
+    out.x = cvt_pk_bf16(any ? v.x / den : 0.0f, any ? v.y / den : 0.0f);
+    out.y = cvt_pk_bf16(any ? v.z / den : 0.0f, any ? v.w / den : 0.0f);
+    *reinterpret_cast<uint2*>(p.out + row * D + d0) = out;
 }
 
 // The chunk form's merge of its key splits: thread c takes the 8 dims ch = c % (D/8) of row
@@ -640,11 +648,11 @@ void launch_decode_d(const AttnParams& p, bool prep, hipStream_t stream) {
 
 namespace {
 
-// Rows of fp32 partials (m, l and head_dim values each) a split workspace holds: 64 splits of
-// the decode form's rows, or one row tile per compute unit of the chunk form (256 on MI355X; a
+// Rows of fp32 partials (m, l and head_dim values each) a split workspace holds: every split
+// of the decode form's 16 rows per kv head, or one row tile per compute unit of the chunk form (256 on MI355X; a
 // plan needs no device).
 size_t workspace_rows(uint32_t n_kv_heads) {
-    constexpr size_t kDecodeRows = 64, kPlanComputeUnits = 256;
+    constexpr size_t kDecodeRows = 16, kPlanComputeUnits = 256;
     return std::max(kAttnMaxSplits * kDecodeRows * n_kv_heads, kPlanComputeUnits * kChunkRows);
 }
 
@@ -695,7 +703,9 @@ bool attention_prep_fits(uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_di
 }
 
 // The decode form's splits: one wave per block of 32 keys (each wave then makes a single
-// round trip to memory for its keys), within kAttnMaxSplits.
+// round trip to memory for its keys), within kAttnMaxSplits - a wave per compute unit for one
+// kv head. Measured against at most 64 (16 heads, one kv head of 512, with the combine): 1000
+// keys 14.0 -> 12.6 us, 8000 32.9 -> 16.8, 30001 93.9 -> 31.0, 262000 759 -> 188 (2.9 TB/s).
 uint32_t decode_splits(uint32_t n_kv_heads, uint32_t keys) {
     (void)n_kv_heads;
     return std::max(1u, std::min(kAttnMaxSplits, (keys + kKeyBlock - 1u) / kKeyBlock));
@@ -790,7 +800,7 @@ void launch_attention(const AttnArgs& a, hipStream_t stream) {
     } else if (p.splits > 1u) {
         const uint64_t rows = static_cast<uint64_t>(a.L) * a.n_heads;
         HYP_REQUIRE(rows <= 0x7fffffffull, HYP_STATUS_INVALID_ARGUMENT, "attention: too many rows to combine");
-        const dim3 grid(static_cast<uint32_t>(rows), a.head_dim > 256u ? a.head_dim / 256u : 1u);
+        const dim3 grid(static_cast<uint32_t>(rows), a.head_dim / 64u);
         switch (a.head_dim) {
             case 64: hipLaunchKernelGGL(attn_combine_kernel<64>, grid, dim3(kAttnThreads), 0, stream, p); break;
             case 128: hipLaunchKernelGGL(attn_combine_kernel<128>, grid, dim3(kAttnThreads), 0, stream, p); break;

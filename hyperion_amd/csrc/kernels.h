@@ -152,7 +152,7 @@ void launch_sample_stochastic(const uint16_t* logits, uint32_t vocab, void* work
 // Attention (forward.cc:376-508) over a KV cache prefix and the current chunk; see
 // attention.hip. Calls that leave compute units idle split the keys; the partial sums need
 // attention_workspace_bytes.
-constexpr uint32_t kAttnMaxSplits = 64;
+constexpr uint32_t kAttnMaxSplits = 256;
 struct AttnPrepareArgs;
 struct AttnArgs {
     const uint16_t* q;         // [L][n_heads][head_dim]

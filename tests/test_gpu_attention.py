@@ -97,6 +97,10 @@ CHUNK_CASES = [
     (5, 16, 1, 512, 700, 650, 650, 0, True),      # many key splits of one partial tile
     (70, 16, 1, 512, 2200, 2100, 2100, 0, True),  # splits whose causal end is inside the last block
     (64, 16, 1, 512, 16, 33, 16, 0, False),       # a ring of half a key block
+    # the decode form with more than 64 splits: fewer in use than in the grid; the first ones
+    # wholly behind the window
+    (1, 4, 1, 64, 9000, 8700, 8700, 0, True),
+    (2, 16, 2, 128, 9000, 9990, 8500, 300, True),
 ]
 
 
