@@ -65,6 +65,7 @@ __device__ __forceinline__ float2 rope_angle(uint32_t pos, uint32_t i, uint32_t 
 // (norm_row_lanes8) and all 64 lanes in its RoPE. The same bits.
 __global__ __launch_bounds__(kThreads) void attn_prepare_head_kernel(PrepareParams p) {
     __shared__ __attribute__((aligned(16))) uint16_t head[kWaves][kMaxHeadDim];
+    __shared__ float2 angle[kMaxHeadDim / 2u];
     const uint32_t t = blockIdx.x;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = threadIdx.x >> 6;
@@ -78,16 +79,12 @@ __global__ __launch_bounds__(kThreads) void attn_prepare_head_kernel(PreparePara
     uint16_t* hb = head[wave];
     uint16_t* dst = nullptr;
 
-    // This lane's pairs i = lane + 64 j: their (cos, sin), looked up or computed.
-    float2 cs[kMaxHeadDim / 128];
-#pragma unroll
-    for (uint32_t j = 0; j < kMaxHeadDim / 128; ++j) {
-        const uint32_t i = lane + 64u * j;
-        cs[j] = make_float2(1.0f, 0.0f);
-        if (active && i < half) {
-            cs[j] = p.rope_cs != nullptr ? p.rope_cs[static_cast<size_t>(pos) * half + i]
-                                         : rope_angle(pos, i, D, p.rotated, p.base);
-        }
+    // The token's (cos, sin), one pair per thread, looked up or computed: every head of the
+    // workgroup shares them (a wave computing its own took 2 to 4 fp64 angles per lane: one
+    // token of a 12B sliding layer 5.9 -> 4.3 us, of a global one 6.8 -> 4.9).
+    for (uint32_t i = threadIdx.x; i < half; i += kThreads) {
+        angle[i] = p.rope_cs != nullptr ? p.rope_cs[static_cast<size_t>(pos) * half + i]
+                                        : rope_angle(pos, i, D, p.rotated, p.base);
     }
     if (active) {
         // 8 values per lane (norm_row_lanes8): every lane of the wave in the norm.
@@ -118,7 +115,7 @@ __global__ __launch_bounds__(kThreads) void attn_prepare_head_kernel(PreparePara
         norm_row_lanes8(xc, &wc, D, p.eps, lane);
         if (has) reinterpret_cast<uint4*>(hb)[lane] = xc;
     }
-    __syncthreads();   // the staged head is visible to every lane of its wave
+    __syncthreads();   // the staged head is visible to every lane of its wave, the angles to all
     if (active) {
 #pragma unroll
         for (uint32_t j = 0; j < kMaxHeadDim / 128; ++j) {
@@ -126,10 +123,11 @@ __global__ __launch_bounds__(kThreads) void attn_prepare_head_kernel(PreparePara
             if (i >= half) break;
             const float x1 = bf16_bits_to_f32(hb[i]);
             const float x2 = bf16_bits_to_f32(hb[i + half]);
-            const float a1 = x1 * cs[j].x;
-            const float a2 = x2 * cs[j].y;
-            const float b1 = x1 * cs[j].y;
-            const float b2 = x2 * cs[j].x;
+            const float2 cs = angle[i];
+            const float a1 = x1 * cs.x;
+            const float a2 = x2 * cs.y;
+            const float b1 = x1 * cs.y;
+            const float b2 = x2 * cs.x;
             dst[i] = f32_to_bf16_bits(a1 - a2);
             dst[i + half] = f32_to_bf16_bits(b1 + b2);
         }
@@ -153,6 +151,7 @@ __global__ __launch_bounds__(kThreads) void attn_prepare_kernel(PrepareParams p)
     constexpr uint32_t kHalfChunks = kHalf / 8u;
     constexpr uint32_t kRopeRows = 64u / kHalfChunks;   // rows one RoPE pass covers
     __shared__ __attribute__((aligned(16))) uint16_t stage[kWaves][kR * D];
+    __shared__ __attribute__((aligned(16))) float2 angles[kWaves][kHalf];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t per_tok = p.H + 2u * p.KVH;
@@ -209,28 +208,35 @@ __global__ __launch_bounds__(kThreads) void attn_prepare_kernel(PrepareParams p)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // RoPE of the staged q and K rows: a lane takes 8 consecutive pairs (i, i + D/2).
-    {
-        const uint32_t c = lane % kHalfChunks;
-        for (uint32_t rr = lane / kHalfChunks; rr < kR; rr += kRopeRows) {
-            uint32_t tr, kr, hr;
-            bool ar;
-            row_of(row0 + rr, tr, kr, hr, ar);
-            if (!ar || kr == 2u) continue;
-            const uint32_t pos = base_pos + tr;
-            float2 cs8[8];
-            if (p.rope_cs != nullptr) {
-                const float4* t4 = reinterpret_cast<const float4*>(p.rope_cs + static_cast<size_t>(pos) * kHalf + c * 8u);
+    // RoPE of the staged q and K rows, a token at a time (the wave's rows lie in one or two
+    // tokens on the 12B): its (cos, sin) in LDS, a pair or a few per lane, looked up or
+    // computed; then a lane takes 8 consecutive pairs (i, i + D/2) of a row. (Angles formed per
+    // row, 8 fp64 ones per lane and pass, bounded the kernel: 1000 tokens of a sliding layer
+    // 31.4 -> 14.8 us, 2048 of a global one 69.8 -> 33.5; read from a table 24.3 -> 17.9 (1111 tokens, sliding).)
+    const uint32_t row_end = min(row0 + kR, total);
+    const uint32_t c = lane % kHalfChunks;
+    for (uint32_t tok = row0 / per_tok; tok * per_tok < row_end; ++tok) {
+        const uint32_t pos = base_pos + tok;
+        float2* cs = angles[wave];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float4 v = t4[e];
-                    cs8[2 * e] = make_float2(v.x, v.y);
-                    cs8[2 * e + 1] = make_float2(v.z, v.w);
-                }
-            } else {
+        for (uint32_t i = lane; i < kHalf; i += 64u) {
+            cs[i] = p.rope_cs != nullptr ? p.rope_cs[static_cast<size_t>(pos) * kHalf + i]
+                                         : rope_angle(pos, i, D, p.rotated, p.base);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        float2 cs8[8];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) cs8[e] = rope_angle(pos, c * 8u + e, D, p.rotated, p.base);
-            }
+        for (int e = 0; e < 4; ++e) {
+            const float4 v = reinterpret_cast<const float4*>(cs + c * 8u)[e];
+            cs8[2 * e] = make_float2(v.x, v.y);
+            cs8[2 * e + 1] = make_float2(v.z, v.w);
+        }
+        const uint32_t first = max(row0, tok * per_tok) - row0;
+        const uint32_t end = max(min(row_end, (tok + 1u) * per_tok - p.KVH), row0) - row0;   // its V rows follow
+        for (uint32_t rr = first + lane / kHalfChunks; rr < end; rr += kRopeRows) {
+            if (tok < p.first_cached && row0 + rr - tok * per_tok >= p.H) continue;   // a K row not cached
             uint4* lo = reinterpret_cast<uint4*>(sw + rr * D + c * 8u);
             uint4* hi = reinterpret_cast<uint4*>(sw + rr * D + kHalf + c * 8u);
             const uint4 a = *lo;
@@ -261,10 +267,10 @@ __global__ __launch_bounds__(kThreads) void attn_prepare_kernel(PrepareParams p)
             *lo = make_uint4(ow[0], ow[1], ow[2], ow[3]);
             *hi = make_uint4(pw[0], pw[1], pw[2], pw[3]);
         }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     if (active && kind != 2u) {
         uint4* dst = kind == 0u ? reinterpret_cast<uint4*>(p.q + (static_cast<size_t>(t) * p.H + hd) * D + u * 64u)
                                 : reinterpret_cast<uint4*>(p.cache_k + slot_row + u * 64u);
