@@ -10,19 +10,18 @@
 // tiled resident layout's (q4_layout.h): for a 16-column tile and a pair of groups,
 // lane (j, kb) loads one 16-byte entry holding words 2kb, 2kb+1 of row j for both
 // groups, i.e. exactly its B values for the pair's four 32-k MFMA steps. So:
-//  * A workgroup (4 waves) computes a (16*MT) x (64*NT) output tile; wave w owns
-//    columns [16*NT*w, 16*NT*(w+1)) for every row, so each weight is dequantized by
-//    exactly one wave, in registers: code -> fp32 -> fma(scale, q, bias) -> one
-//    rounding to bf16 (v_cvt_pk_bf16_f32), the MLX dequantized value.
-//  * The k loop advances one pair of groups (128 k) per iteration. X tiles of
-//    (16*MT) x 128 bf16 go straight from HBM to LDS (16-byte buffer loads with the LDS
-//    as destination, no VGPRs), double buffered with one barrier per iteration; the
-//    next tile and the next pair's weights are in flight while the current pair
-//    computes. LDS rows are 256 bytes with their 16-byte chunks XOR-swizzled by
-//    (row % 16), so the 16 rows an A-fragment read touches hit distinct banks.
-//  * Within an iteration the B fragments of k-step s+1 are dequantized while the
-//    MFMAs of step s run, and each step's A fragments are read from LDS in one
-//    batch ahead of its MFMAs.
+//  * A workgroup (8 waves) computes a (16*MT) x 256 output tile (MT = 8 or 16); each wave owns
+//    32 columns for every row, so each weight is dequantized by exactly one wave, in
+//    registers: code -> fp32 -> fma(scale, q, bias) -> one rounding to bf16
+//    (v_cvt_pk_bf16_f32), the MLX dequantized value.
+//  * The k loop advances one group (64 k) per iteration. X tiles of (16*MT) x 64 bf16 go
+//    straight from HBM to LDS (16-byte buffer loads with the LDS as destination, no
+//    VGPRs) through a ring of stages, with the chunks of a row XOR-swizzled so that the 16
+//    rows an A-fragment read touches hit distinct banks; later stages and weights are in
+//    flight while the current group computes.
+//  * The B fragments of the next k-step are dequantized while the MFMAs of one run, and A
+//    fragments are read from LDS a unit ahead of their MFMAs.
+//  * Calls of few rows have a kernel of their own (q4_gemm_few_kernel).
 //  * Workgroup ids are remapped so each XCD (ids are dealt round-robin over the 8 XCDs)
 //    gets a contiguous run of tiles that share X rows, keeping the X block in that
 //    XCD's L2.
@@ -43,12 +42,10 @@ namespace {
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
-constexpr int kWaves = kThreads / 64;
-constexpr int kPairK = 128;                 // k per iteration (two groups)
-constexpr int kRowBytes = kPairK * 2;       // one LDS row of an X tile
+constexpr int kPairK = 128;                 // k of a pair of groups
 
 // One projection of a (possibly grouped) launch: its workgroup column tiles are the
-// global column tiles [tn_begin, tn_begin + ceil(n / 128)).
+// global column tiles [tn_begin, tn_begin + ceil(n / tile width)).
 struct GemmSegment {
     const uint4* codes;   // tiled codes (q4_layout.h)
     const uint2* sb;      // tiled scales and biases
@@ -72,7 +69,7 @@ struct GemmParams {
     uint32_t pairs;       // ceil(k / 128)
     uint32_t tiles_n;     // workgroup column tiles over all segments
     uint32_t tiles_total;
-    // Split k (pair-step kernel): ksplit workgroups share an output tile, each covering
+    // Split k: ksplit workgroups share an output tile, each covering
     // pairs_per_split pairs, and write fp32 partials to partial[ksplit][m][n_total].
     uint32_t ksplit;
     uint32_t pairs_per_split;
@@ -147,44 +144,6 @@ __device__ __forceinline__ void load_b(const R& wr, const uint32_t (&c_off)[NT],
             uint4, __builtin_amdgcn_raw_buffer_load_b128(wr.c[nt & 1], c_off[nt], pair * 1024u, 0));
         raw.sb[nt] = __builtin_bit_cast(
             uint2, __builtin_amdgcn_raw_buffer_load_b64(wr.s[nt & 1], s_off[nt], pair * 128u, 0));
-    }
-}
-
-// The MFMAs of k-step S over all M tiles; A fragments come from the LDS tile
-// (swizzled rows: logical chunk c of row r sits at chunk c ^ (r % 16)).
-template <int MT, int NT, int S>
-__device__ __forceinline__ void mfma_step(const uint8_t* xb, uint32_t lane, const bf16x8_t (&b)[NT],
-                                          f32x4_t (&acc)[MT][NT]) {
-    const uint32_t i = lane & 15u;
-    const uint32_t kb = lane >> 4;
-    // This lane's 8 values: group S/2, word 2kb + S%2 of the pair, i.e. logical chunk c.
-    const uint32_t c = (S / 2) * 8u + 2u * kb + (S % 2);
-    const uint8_t* row = xb + i * kRowBytes + ((c ^ i) << 4);
-    constexpr int kHalf = MT / 2;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        bf16x8_t a[kHalf];
-#pragma unroll
-        for (int mt = 0; mt < kHalf; ++mt)
-            a[mt] = *reinterpret_cast<const bf16x8_t*>(row + (h * kHalf + mt) * 16u * kRowBytes);
-#pragma unroll
-        for (int mt = 0; mt < kHalf; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-                acc[h * kHalf + mt][nt] =
-                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], b[nt], acc[h * kHalf + mt][nt], 0, 0, 0);
-    }
-    // Scheduling hint for this region (the dequantization of the next step, issued just
-    // before, and these MFMAs): the first half's A reads, then one MFMA followed by
-    // kValu VALU ops throughout, with the second half's A reads after the first MFMAs.
-    constexpr int kMfma = MT * NT;
-    constexpr int kValu = (NT * 25 + kMfma - 1) / kMfma;   // dequant ops of a step per MFMA
-    __builtin_amdgcn_sched_group_barrier(0x100, kHalf, 0);   // DS read
-#pragma unroll
-    for (int t = 0; t < kMfma; ++t) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);       // MFMA
-        __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);   // VALU
-        if (t == 1) __builtin_amdgcn_sched_group_barrier(0x100, kHalf, 0);
     }
 }
 
@@ -336,171 +295,10 @@ __device__ __forceinline__ void stage_out(uint8_t* xs, uint32_t out_row, uint32_
             }
 }
 
-template <int MT, int NT, bool ODD, bool DUAL>
-__global__ __launch_bounds__(kThreads) void q4_gemm_kernel(GemmParams p) {
-    static_assert(!DUAL || NT == 2, "a dual launch pairs one gate and one up tile per wave");
-    constexpr int kOut = DUAL ? 1 : NT;   // output column tiles per wave
-    constexpr int BM = 16 * MT;
-    constexpr int kTileBytes = BM * kRowBytes;
-    constexpr int kXLoads = BM / 4 / kWaves;   // 1 KB direct loads per wave per X tile
-    extern __shared__ __attribute__((aligned(16))) uint8_t xs[];   // [2][BM][256 B]
-
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-
-    // XCD-aware tile order: XCD x = blockIdx % 8 runs tiles [start_x, start_x + count_x).
-    const uint32_t bid = blockIdx.x;
-    const uint32_t xcd = bid & 7u;
-    const uint32_t slot = bid >> 3;
-    const uint32_t ext_total = p.tiles_total * p.ksplit;
-    const uint32_t per = ext_total >> 3;
-    const uint32_t rem = ext_total & 7u;
-    const uint32_t ext = xcd * per + min(xcd, rem) + slot;
-    const uint32_t kz = ext / p.tiles_total;          // this workgroup's k split
-    const uint32_t tile = ext - kz * p.tiles_total;
-    const uint32_t tm = tile / p.tiles_n;
-    const SegView sv = view_of<DUAL>(p, tile - tm * p.tiles_n);
-    const uint32_t m0 = tm * BM;
-    const uint32_t n0 = sv.tn * (kWaves * 16u * kOut);
-    const uint32_t tile16_0 = n0 / 16u + wave * kOut;
-
-    const uint32_t k = p.k;
-    const uint32_t pairs = p.pairs;
-
-    // X staging: load t of wave w covers tile rows 4 (w kXLoads + t) .. +3; lane l fills
-    // LDS chunk (l % 16) of row r = 4 (w kXLoads + t) + l / 16 with the row's logical
-    // chunk (l % 16) ^ (r % 16). kXLoads is a multiple of 4, so r % 16 = (4 t + l / 16)
-    // % 16. Each load's lane offset is set up once; the pair is a scalar offset. Rows past
-    // m get an offset past the buffer resource (m * k * 2 bytes) and load zeros; so do the
-    // chunks past k of an odd group count (ODD: the last pair's second group).
-    static_assert(kXLoads % 4 == 0, "swizzle period");
-    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(p.x), static_cast<short>(0), static_cast<int>(p.m * k * 2u), 0x00020000);
-    const uint32_t lh = lane >> 4;
-    uint32_t xoff[kXLoads];
-    uint32_t xchunk[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) xchunk[t] = (lane & 15u) ^ ((4u * t + lh) & 15u);
-#pragma unroll
-    for (int t = 0; t < kXLoads; ++t) {
-        const uint32_t row = m0 + 4u * (wave * kXLoads + t) + lh;
-        xoff[t] = row < p.m ? row * k * 2u + xchunk[t % 4] * 16u : 0x80000000u;
-    }
-    auto load_x = [&](uint32_t pair, uint8_t* buf) {
-#pragma unroll
-        for (int t = 0; t < kXLoads; ++t) {
-            uint32_t off = xoff[t];
-            if (ODD && pair * kPairK + xchunk[t % 4] * 8u >= k) off = 0x80000000u;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                xr, (__attribute__((address_space(3))) void*)(buf + (wave * kXLoads + t) * 1024u), 16,
-                static_cast<int>(off), static_cast<int>(pair * kPairK * 2u), 0, 0);
-        }
-    };
-
-    // Weights: column tile (tile16_0 + nt) (DUAL: tile tile16_0 of the gate, then of up),
-    // clamped to the last tile (columns past n are computed, never stored).
-    const WeightRsrc wr = weight_rsrc<DUAL>(p, sv);
-    uint32_t c_off[NT];
-    uint32_t s_off[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-        const uint32_t t16 = min(tile16_0 + (DUAL ? 0u : static_cast<uint32_t>(nt)), sv.row_tiles - 1u);
-        c_off[nt] = (t16 * pairs * 64u + lane) * 16u;
-        s_off[nt] = (t16 * pairs * 16u + (lane & 15u)) * 8u;
-    }
-
-    f32x4_t acc[MT][NT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-
-    // This workgroup's pairs [p0, p1) (all of them without split k).
-    const uint32_t p0 = kz * p.pairs_per_split;
-    const uint32_t p1 = min(p0 + p.pairs_per_split, pairs);
-
-    BRaw<NT> braw, bnext;
-    load_x(p0, xs);
-    load_b<NT>(wr, c_off, s_off, p0, braw);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-
-    bf16x8_t b0[NT], b1[NT];
-    dequant_step<NT, 0>(braw, b0);
-
-    // The loop body has no branches (branches split the accumulators' live ranges and
-    // cost AGPR copies); the last iteration prefetches its own pair again, harmlessly.
-    for (uint32_t pair = p0; pair < p1; ++pair) {
-        const uint8_t* xb = xs + ((pair - p0) & 1u) * kTileBytes;
-        const uint32_t pn = min(pair + 1u, p1 - 1u);
-        load_x(pn, xs + ((pair - p0 + 1u) & 1u) * kTileBytes);
-        load_b<NT>(wr, c_off, s_off, pn, bnext);
-
-        dequant_step<NT, 1>(braw, b1);
-        mfma_step<MT, NT, 0>(xb, lane, b0, acc);
-        dequant_step<NT, 2>(braw, b0);
-        mfma_step<MT, NT, 1>(xb, lane, b1, acc);
-        dequant_step<NT, 3>(braw, b1);
-        mfma_step<MT, NT, 2>(xb, lane, b0, acc);
-        braw = bnext;
-        dequant_step<NT, 0>(braw, b0);
-        mfma_step<MT, NT, 3>(xb, lane, b1, acc);
-
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-    }
-
-    if (p.ksplit > 1u) {
-        store_partials<MT, NT, kOut, DUAL>(p, sv, kz, m0, n0, wave, lane, acc);
-        return;
-    }
-
-    // Epilogue: the workgroup's (16 MT) x (64 kOut) tile goes through LDS (rows of
-    // 128 kOut bytes plus 32 bytes of padding, so the four row groups a write touches hit
-    // distinct banks) and leaves as 16-byte row segments. acc[mt][nt][r] is tile element
-    // (16 mt + 4 kb + r, 16 kOut wave + 16 nt + j) (DUAL: nt = 0 gate, 1 up of column
-    // 16 wave + j).
-    constexpr uint32_t kOutRow = 128u * kOut + 32u;
-    static_assert(BM * kOutRow + (DUAL ? kGeluTableBytes : 0u) <= 2u * kTileBytes,
-                  "output staging exceeds the X buffers");
-    uint16_t* tab = reinterpret_cast<uint16_t*>(xs + BM * kOutRow);
-    __syncthreads();
-    if constexpr (DUAL) {
-        build_gelu_table(tab, tid, kThreads);
-        __syncthreads();
-    }
-    stage_out<MT, NT, kOut, DUAL>(xs, kOutRow, wave, lane, acc, tab);
-    __syncthreads();
-    constexpr uint32_t kCols = 64u * kOut;
-    constexpr uint32_t kChunks = kCols / 8u;                  // 16-byte chunks per row
-    constexpr uint32_t kRowsPerPass = kThreads / kChunks;
-    const uint32_t ch = threadIdx.x % kChunks;
-    const uint32_t col0 = n0 + ch * 8u;
-    if ((sv.n & 7u) == 0u && (reinterpret_cast<uintptr_t>(sv.y) & 15u) == 0u) {
-        for (uint32_t r = threadIdx.x / kChunks; r < BM; r += kRowsPerPass) {
-            const uint32_t row = m0 + r;
-            if (row < p.m && col0 < sv.n)
-                *reinterpret_cast<uint4*>(sv.y + static_cast<size_t>(row) * sv.n + col0) =
-                    *reinterpret_cast<const uint4*>(xs + r * kOutRow + ch * 16u);
-        }
-    } else {
-        for (uint32_t r = threadIdx.x / kChunks; r < BM; r += kRowsPerPass) {
-            const uint32_t row = m0 + r;
-            if (row >= p.m) continue;
-            for (uint32_t c = 0; c < 8u; ++c)
-                if (col0 + c < sv.n)
-                    sv.y[static_cast<size_t>(row) * sv.n + col0 + c] =
-                        *reinterpret_cast<const uint16_t*>(xs + r * kOutRow + ch * 16u + c * 2u);
-        }
-    }
-}
-
-// ---- group-step variant: 256-row tiles, one group (64 k) per iteration ---------------
+// ---- tile kernel, one group (64 k) per iteration ----------------------------------------
 //
-// The same scheme with 16 row tiles per wave (each dequantized B fragment feeds 16 MFMAs
-// instead of 8) and 64-k iterations, so two workgroups still fit a CU: X stages of
-// 256 rows x 128 bytes (chunks swizzled by row % 16, see g_read_a), double buffered; the raw weights of
+// 16 or 8 row tiles per wave (each dequantized B fragment feeds that many MFMAs). X stages
+// are 16 MT rows x 128 bytes (chunks swizzled by row % 16, see g_read_a); the raw weights of
 // a group are half of each 16-byte entry (plus its scale word), loaded two groups ahead.
 // k-step s of a group uses word 2 kb + s of the lane's entry, and the A fragments the
 // same k chunk.
@@ -773,7 +571,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2))) 
         return;
     }
 
-    // Epilogue through LDS as in q4_gemm_kernel (rows of 32 kOut W bytes plus 32 of padding).
+    // Epilogue: the tile goes through LDS (rows of 32 kOut W bytes plus 32 of padding, so the four
+    // row groups a write touches hit distinct banks) and leaves as 16-byte row segments.
     constexpr uint32_t kOutRow = 32u * kOut * W + 32u;
     static_assert(BM * kOutRow <= g_lds_bytes<MT, NT, W>(), "output staging exceeds the X ring");
     __syncthreads();
@@ -1014,14 +813,13 @@ size_t max_lds_per_block() {
     return cached;
 }
 
-constexpr uint32_t kTileCols = 128u;   // workgroup tile width of the pair-step kernel (NT = 2)
-
 // Column tiles of `tile_cols` output columns: each segment's first global tile and the
 // total (a dual launch tiles the gate's columns only; up rides along).
 void retile(GemmParams& p, uint32_t tile_cols) {
     if (p.dual != 0u) {
         p.seg[0].tn_begin = 0u;
         p.tiles_n = (p.seg[0].n + tile_cols - 1u) / tile_cols;
+        p.seg[1].tn_begin = p.tiles_n;   // past every tile: view_of takes the gate's segment
         return;
     }
     uint32_t tn = 0;
@@ -1030,30 +828,6 @@ void retile(GemmParams& p, uint32_t tile_cols) {
         tn += (p.seg[i].n + tile_cols - 1u) / tile_cols;
     }
     p.tiles_n = tn;
-}
-
-template <int MT, int NT, bool DUAL>
-void launch_t(GemmParams p, hipStream_t stream) {
-    retile(p, kWaves * 16u * (DUAL ? 1u : NT));
-    const bool odd = ((p.k / 64u) & 1u) != 0u;
-    auto kernel = odd ? q4_gemm_kernel<MT, NT, true, DUAL> : q4_gemm_kernel<MT, NT, false, DUAL>;
-    const size_t lds = 2u * 16u * MT * kRowBytes;
-    HYP_REQUIRE(lds <= max_lds_per_block(), HYP_STATUS_INTERNAL, "gemm: X tiles exceed the device's LDS");
-    if (lds > 65536u) {
-        static thread_local int configured_device = -1;
-        int dev = 0;
-        HYP_HIP_CHECK(hipGetDevice(&dev));
-        if (configured_device != dev) {
-            HYP_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(q4_gemm_kernel<MT, NT, true, DUAL>),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-            HYP_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(q4_gemm_kernel<MT, NT, false, DUAL>),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-            configured_device = dev;
-        }
-    }
-    const uint32_t tiles_m = (p.m + 16u * MT - 1u) / (16u * MT);
-    p.tiles_total = p.tiles_n * tiles_m;
-    hipLaunchKernelGGL(kernel, dim3(p.tiles_total * p.ksplit), dim3(kThreads), lds, stream, p);
 }
 
 template <int MT, int NT, int W, bool DUAL>
@@ -1148,7 +922,6 @@ GemmParams group_params(const Q4Matrix* const* ws, uint16_t* const* ys, uint32_t
     HYP_REQUIRE(static_cast<uint64_t>(m) * k * 2u < (1ull << 31), HYP_STATUS_INVALID_ARGUMENT,
                 "gemm: x is 2 GiB or larger");
     GemmParams p{};
-    uint32_t tn = 0;
     uint32_t n_total = 0;
     for (uint32_t i = 0; i < count; ++i) {
         const Q4Matrix& w = *ws[i];
@@ -1158,8 +931,7 @@ GemmParams group_params(const Q4Matrix* const* ws, uint16_t* const* ys, uint32_t
         const TiledDims d = TiledDims::of(w.n, w.k);
         HYP_REQUIRE(d.code_bytes() < (1ull << 31), HYP_STATUS_INVALID_ARGUMENT, "gemm: weights of 2 GiB or more");
         p.seg[i] = GemmSegment{w.codes, w.sb, ys[i], w.n, d.tiles, static_cast<uint32_t>(d.code_bytes()),
-                               static_cast<uint32_t>(d.sb_bytes()), tn, n_total};
-        tn += (w.n + kTileCols - 1u) / kTileCols;
+                               static_cast<uint32_t>(d.sb_bytes()), 0u, n_total};
         n_total += w.n;
     }
     p.nseg = count;
@@ -1167,7 +939,7 @@ GemmParams group_params(const Q4Matrix* const* ws, uint16_t* const* ys, uint32_t
     p.m = m;
     p.k = k;
     p.pairs = TiledDims::of(16u, k).pairs;
-    p.tiles_n = tn;
+    p.tiles_n = 0u;   // (retile, for the chosen kernel)
     p.ksplit = 1u;
     p.pairs_per_split = p.pairs;
     p.n_total = n_total;
@@ -1176,9 +948,11 @@ GemmParams group_params(const Q4Matrix* const* ws, uint16_t* const* ys, uint32_t
     return p;
 }
 
-// The three GEMM kernels by workgroup tile.
+// Bytes of the fixed scratch of launch_q4_gemm_noalloc (below).
+constexpr size_t kNoAllocScratchBytes = size_t{64} << 20;
+
+// The tile kernels.
 enum class GemmKernel : uint32_t {
-    kPair128 = 0,    // q4_gemm_kernel<8, 2>: 128 x 128, pair step, two workgroups per CU
     kGroup128 = 1,   // q4_gemm_g_kernel<8, 2, 8>: 128 x 256, group step, one per CU
     kGroup256 = 2,   // q4_gemm_g_kernel<16, 2, 8>: 256 x 256, group step, one per CU
 };
@@ -1191,7 +965,6 @@ struct GemmChoice {
 template <bool DUAL>
 void launch_kernel(GemmParams& p, GemmKernel kernel, hipStream_t stream) {
     switch (kernel) {
-        case GemmKernel::kPair128: launch_t<8, 2, DUAL>(p, stream); break;
         case GemmKernel::kGroup128: launch_g<8, 2, kGroupWaves, DUAL>(p, stream); break;
         case GemmKernel::kGroup256: launch_g<16, 2, kGroupWaves, DUAL>(p, stream); break;
         default: throw NativeError(HYP_STATUS_INTERNAL, "gemm: unsupported kernel");
@@ -1222,29 +995,58 @@ uint32_t fill_split(const GemmParams& p, uint64_t tiles, uint64_t cus) {
     return s;
 }
 
-// Kernel and split per call. From a sweep of the seven projections and the grouped q/k/v
-// at m = 512, 1024 and 2048 on seeded random data (all three kernels, 1-4 splits), these
-// rules pick the fastest configuration or one within 5% of it:
-//  * the 256 x 256 kernel when its grid fills 90% of the CUs (gate/up at m >= 1024, the
-//    grouped q/k/v at 2048), or does so split when k is long (down at m = 1024: 4 splits,
-//    125 us against 192 on the pair-step kernel; at 2048: 2 splits, 215 against 226);
-//  * else the 128 x 256 kernel, split to fill the CUs, when that reaches 60% of them
-//    (gate at m = 512: 71 us against 81; o at 2048: 67 against 76);
-//  * else the 128 x 128 pair-step kernel, split likewise (k [2048, 3840] at m = 512, 4
-//    splits: 33 us against 34-36).
-GemmChoice choose_gemm(const GemmParams& p) {
+// k splits that fill the compute units, at most 4 (the split count of small launches, and the
+// bound that the fixed scratch of launch_q4_gemm_noalloc is checked against).
+uint32_t filling_split(const GemmParams& p) {
     const uint64_t cus = device_compute_units();
     const uint64_t big = gemm_tiles(p, 256u, 256u);
-    if (big * 10u >= cus * 9u) return {GemmKernel::kGroup256, 1u};
+    if (big * 10u >= cus * 9u) return 1u;
     if (p.pairs >= 64u) {
         const uint32_t s = fill_split(p, big, cus);
-        if (big * s * 10u >= cus * 9u) return {GemmKernel::kGroup256, s};
+        if (big * s * 10u >= cus * 9u) return s;
     }
     const uint64_t mid = gemm_tiles(p, 128u, 256u);
     const uint32_t s = fill_split(p, mid, cus);
-    if (mid * s * 10u >= cus * 6u) return {GemmKernel::kGroup128, s};
-    const uint64_t pair = gemm_tiles(p, 128u, 128u);
-    return {GemmKernel::kPair128, fill_split(p, pair, cus)};
+    if (mid * s * 10u >= cus * 6u) return s;
+    return fill_split(p, gemm_tiles(p, 128u, 128u), cus);
+}
+
+// Kernel and split per call: the ones with the least estimated time,
+//   4 us + rounds of one workgroup per compute unit x groups per split x time per group
+//   + (split) 4 us + the partials' write and read at 5.5 TB/s,
+// where a group (64 k) of the 128-row kernel takes 0.72 us, of the 256-row kernel 1.3 us, and
+// up to 0.95 and 1.65 us as the grid covers the compute units. From a sweep of the projections
+// at 100 to 2048 rows, all splits to 12, which the estimate meets within about 10%: the ragged
+// grids are what it is for, where filling the compute units by splitting runs into a second
+// round. Against that rule (us): down [3840, 15360] 203 rows 61.8 -> 43.8, 700 rows 148.6 ->
+// 111.6, 1111 rows 194 -> 160; q/k/v [8192, 3840] 300 rows 56.0 -> 42.4, 700 rows 77.6 -> 54.4; o
+// [3840, 4096] 700 rows 58.9 -> 43.4; [15360, 3840] 300 rows 74.1 -> 54.0. The 128 x 128
+// pair-step kernel is at best equal to the 128 x 256 one at the same split (two workgroups per
+// compute unit, each waiting for its loads), and kept for narrow outputs of at most 128 columns.
+GemmChoice choose_gemm(const GemmParams& p) {
+    const uint64_t cus = device_compute_units();
+    const uint32_t most = filling_split(p);
+    GemmChoice best{GemmKernel::kGroup128, 1u};
+    double best_us = 1e30;
+    for (const GemmKernel kernel : {GemmKernel::kGroup256, GemmKernel::kGroup128}) {
+        const bool big = kernel == GemmKernel::kGroup256;
+        const uint64_t tiles = gemm_tiles(p, big ? 256u : 128u, 256u);
+        for (uint32_t s = 1u; s <= 16u && (p.pairs + s - 1u) / s >= 3u; ++s) {
+            const uint64_t bytes = static_cast<uint64_t>(s) * p.m * p.n_total * sizeof(float);
+            if (s > most && bytes > kNoAllocScratchBytes) break;   // larger partials only where filling took them
+            const uint64_t grid = tiles * s;
+            const double cover = std::min(1.0, static_cast<double>(grid) / cus);
+            const double full = std::max(0.0, 2.0 * cover - 1.0);
+            const double group = big ? 1.3 + 0.35 * full : 0.72 + 0.23 * full;
+            double us = 4.0 + static_cast<double>((grid + cus - 1u) / cus) * (2u * ((p.pairs + s - 1u) / s)) * group;
+            if (s > 1u) us += 4.0 + 2.0 * bytes / 5.5e6;
+            if (us < best_us) {
+                best_us = us;
+                best = {kernel, s};
+            }
+        }
+    }
+    return best;
 }
 
 // Where the split-k partials of one call live: a stream-ordered temporary
@@ -1309,7 +1111,6 @@ void launch_split(GemmParams& p, GemmKernel kernel, uint32_t ksplit, hipStream_t
 // so that path allocates nothing. Each device holds its own copy (64 MiB) from module
 // load until the process ends; every call on one device shares it, so calls that
 // overlap on one device (e.g. on two streams) race.
-constexpr size_t kNoAllocScratchBytes = size_t{64} << 20;
 static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -1368,6 +1169,11 @@ void launch_q4_gemm_noalloc(const Q4Matrix& w, const uint16_t* x, uint32_t m, ui
     // The same kernel and split as launch_q4_gemm.
     if (few_rows(p)) return launch_few(p, stream);
     const GemmChoice c = choose_gemm(p);
+    const uint64_t filled = static_cast<uint64_t>(filling_split(p)) * m * p.n_total * sizeof(float);
+    HYP_REQUIRE(filling_split(p) == 1u || filled <= kNoAllocScratchBytes, HYP_STATUS_INVALID_ARGUMENT,
+                "gemm: this call's k splits may need " + std::to_string(filled) +
+                    " bytes of partial sums; the no-allocation scratch holds " + std::to_string(kNoAllocScratchBytes) +
+                    " bytes");
     SplitWorkspace wsp;
     wsp.fixed = noalloc_scratch();
     wsp.fixed_bytes = kNoAllocScratchBytes;
