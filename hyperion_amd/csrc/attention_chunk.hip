@@ -21,10 +21,14 @@
 //    each tile in the shadow of the products before its own. At head_dim 512 O is in
 //    accumulation registers (three instructions a value), and is rescaled only when some
 //    row's maximum has grown by more than 2^kRescaleLog2 since the last time. The largest
-//    probability is then no longer the exact 1 of a running maximum, which by itself made
-//    the result's error against fp64 0.8% larger; so half of the probabilities (the first 16
-//    keys of a block) enter as two bf16 terms, which makes it 1.5% smaller (all of them: 4%
-//    smaller, at 341 against 311 us on the first case below, 251 without any).
+//    probability is then no longer the exact 1 of a running maximum: rounded to bf16 against an
+//    unrounded denominator it would leave a row that one key dominates an error of 2.3e-3
+//    where the running maximum's is 1.7e-3 (128 keys, the key 4 to 8 octaves above those before
+//    it). So every probability enters as two bf16 terms (1.66e-3 there, and 2% below the
+//    running maximum on random rows), at 364 us against 324 with second terms for half of the
+//    keys, on the first case below. A block that outgrows the reference takes its score products
+//    twice: 2048 tokens behind 2048 in 391 us on random rows, 453 with their scores' deviation
+//    four times that, 632 where every block of every row does.
 //  * Operands are read from LDS four products ahead of their use, and the next block's loads
 //    go out between the score products.
 //
@@ -34,7 +38,7 @@
 // wave per SIMD at head_dim 512 the softmax between the two products is exposed. Measured, the
 // whole call with its merge, against 16 rows per wave on 16x16x32 products with V transposed
 // or read behind each product: 16 heads, 2048 tokens behind 2048 at head_dim 512 (one kv head)
-// 1110 -> 311 us (186 -> 663 TFLOP/s); 1000 behind 700 at head_dim 256 (8 kv heads, window 1024)
+// 1110 -> 364 us (186 -> 566 TFLOP/s); 1000 behind 700 at head_dim 256 (8 kv heads, window 1024)
 // 118 -> 44 us. Without the reads ahead of use a third slower.
 #include "attention.h"
 #include "common.h"
@@ -326,11 +330,12 @@ __global__ __launch_bounds__(kThreads, D >= 512u ? 1 : 2) void attn_chunk_kernel
         bf16x8_t pb[2];
 #pragma unroll
         for (int t = 0; t < 2; ++t) pb[t] = round_p(pr + 8 * t);
-        bf16x8_t pl;
+        bf16x8_t pl[2];
         if constexpr (kLazy) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) pr[i] -= bf16_bits_to_f32(__builtin_bit_cast(u16x8_t, pb[0])[i]);
-            pl = round_p(pr);
+            for (int i = 0; i < 16; ++i) pr[i] -= bf16_bits_to_f32(__builtin_bit_cast(u16x8_t, pb[i / 8])[i % 8]);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) pl[t] = round_p(pr + 8 * t);
         } else {
 #pragma unroll
             for (int i = 0; i < 16; ++i) o[0][i] *= alpha;
@@ -344,8 +349,8 @@ __global__ __launch_bounds__(kThreads, D >= 512u ? 1 : 2) void attn_chunk_kernel
         for (uint32_t u = 0; u < kProducts; ++u) {
             __builtin_amdgcn_sched_barrier(0);
             o[u / 2u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[u % kAhead], pb[u % 2u], o[u / 2u], 0, 0, 0);
-            if (kLazy && u % 2u == 0u)
-                o[u / 2u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[u % kAhead], pl, o[u / 2u], 0, 0, 0);
+            if constexpr (kLazy)
+                o[u / 2u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[u % kAhead], pl[u % 2u], o[u / 2u], 0, 0, 0);
             if (u + kAhead < kProducts) vf[u % kAhead] = v_read(stage, u + kAhead);
             if (!kLazy && u / 2u + 1u < kDTiles) {   // the next tile, half of it in each product's shadow
 #pragma unroll

@@ -141,6 +141,49 @@ def test_chunk_kernel_edges(stream, L, H, KVH, D, cap, offset, prefix, window, c
     cache.close()
 
 
+def _running_max_f32(q, k, v, prefix):
+    """Attention of one kv head as the online softmax with an exact running maximum gives it:
+    probabilities against the row's maximum, rounded to bf16 for P V, their sum unrounded."""
+    L, H, D = q.shape
+    s = np.einsum("thd,jd->thj", q.astype(np.float64), k.astype(np.float64)) * np.log2(np.e)
+    s = np.where(np.arange(k.shape[0]) <= prefix + np.arange(L)[:, None, None], s, -np.inf)
+    p = np.exp2(s - s.max(-1, keepdims=True)).astype(np.float32)
+    o = syn.bf16_to_f32(syn.bf16_bits(p)).astype(np.float64) @ v.astype(np.float64)
+    return syn.bf16_bits((o / p.astype(np.float64).sum(-1, keepdims=True)).astype(np.float32))
+
+
+@pytest.mark.parametrize("place", [64 + 5, 64 + 21])
+def test_chunk_dominant_key_precision(stream, place):
+    """A key that outgrows the maximum of the keys before it by 4 to 8 octaves, in either half
+    of a key block, at head_dim 512 (where the output is not rescaled for it): the error against
+    fp64 stays that of the running-maximum form, whose largest probability is an exact 1. The
+    bar is 3% above that form's own error, measured over the 65536 outputs (whose relative
+    standard error is 1 / sqrt(2 x 65536) = 0.3%)."""
+    L, H, D, prefix = 8, 16, 512, 120
+    T = prefix + L
+    rng = np.random.default_rng(place)
+    f = lambda a: syn.bf16_to_f32(syn.bf16_bits(a.astype(np.float32)))  # noqa: E731
+    q, k, v = f(rng.standard_normal((L, H, D)) * 0.02), f(rng.standard_normal((T, D)) * 0.2), f(rng.standard_normal((T, D)))
+    k[:, 0] = 0.0
+    q[:, :, 0] = f(rng.uniform(4.0, 8.0, (L, H)) / np.log2(np.e))
+    k[place] = 0.0
+    k[place, 0] = 1.0
+    say(f"dominant key at {place}")
+    qb, kb, vb = (syn.bf16_bits(a) for a in (q, k, v))
+    ref = O.attention_f64(qb, kb[prefix:, None], vb[prefix:, None], kb[:, None], vb[:, None], prefix, prefix, 0)
+    cache = hy.KvCache(T, 1, D)
+    _fill_cache(cache, kb, vb, stream)
+    qd, out = dev(qb, stream), hy.DeviceArray((L, H, D), np.uint16)
+    hy.call("hyp_attention", qd.ptr, None, None, L, H, cache.handle, prefix, prefix, 0, out.ptr, stream.handle)
+    rel = lambda bits: np.linalg.norm(syn.bf16_to_f32(bits) - ref) / np.linalg.norm(ref)  # noqa: E731
+    got, bar = rel(out.to_host(stream)), rel(_running_max_f32(q, k, v, prefix))
+    say(f"  error {got:.3e}, running-maximum form {bar:.3e}")
+    assert got <= 1.03 * bar
+    for a in (qd, out):
+        a.close()
+    cache.close()
+
+
 def test_kv_cache_write_slots_and_ring_overwrite(stream):
     """Tokens land in slot p % capacity; a write longer than the ring keeps its last
     `capacity` tokens; attention over the written prefix equals attention over the same
