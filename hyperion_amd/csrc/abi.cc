@@ -8,6 +8,7 @@
 #include <cstring>
 #include <filesystem>
 #include <memory>
+#include <mutex>
 #include <new>
 #include <string>
 
@@ -119,6 +120,12 @@ struct HypStreamOpaque {
     [[nodiscard]] void* stoch_workspace() const noexcept {
         return static_cast<uint8_t*>(workspace) + stoch_workspace_offset;
     }
+    // Split partials of the attention chunks enqueued on this stream, made by the first that
+    // splits and grown in stream order. The mutex covers a call's whole enqueue: growing from
+    // another thread frees the buffer behind what is enqueued by then.
+    std::mutex attn_mutex;
+    void* attn_partials = nullptr;
+    size_t attn_partials_bytes = 0;
 };
 
 struct HypEventOpaque {
@@ -286,6 +293,7 @@ HypStatus hyp_stream_destroy(HypStream* stream) {
     if ((*stream)->magic != kStreamMagic) {
         return fail(HYP_STATUS_INVALID_ARGUMENT, "handle magic mismatch (wrong type, freed, or corrupted)");
     }
+    if ((*stream)->attn_partials != nullptr) (void)hipFreeAsync((*stream)->attn_partials, (*stream)->stream);
     hipError_t err = hipStreamDestroy((*stream)->stream);
     // hipFree waits for the device, so work still queued on the stream finishes first.
     const hipError_t ferr = hipFree((*stream)->workspace);
@@ -736,6 +744,21 @@ HypKvCacheOpaque& kv_ref(HypKvCache c) {
     return *c;
 }
 
+// The stream's attention partials, at least `bytes` (attn_mutex held); null when the device has
+// no room for them.
+void* attn_partials(HypStreamOpaque& st, size_t bytes) {
+    if (st.attn_partials_bytes >= bytes) return st.attn_partials;
+    void* grown = nullptr;
+    if (hipMallocAsync(&grown, bytes, st.stream) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (st.attn_partials != nullptr) HYP_HIP_CHECK(hipFreeAsync(st.attn_partials, st.stream));
+    st.attn_partials = grown;
+    st.attn_partials_bytes = bytes;
+    return grown;
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0u; }
 }  // namespace
 
@@ -799,6 +822,29 @@ HypStatus hyp_attention(const void* q, const void* k, const void* v, uint32_t L,
         a.window = window;
         a.workspace = c.workspace.data();
         a.workspace_bytes = c.workspace.bytes();
+        // Calls on several streams may read one cache at once, so a chunk's partials are the
+        // stream's own. A recorded chunk replays on any stream: it runs unsplit, except for
+        // at most 64 query rows per kv head, which split in the handle's workspace as the
+        // decode form does (a long context on one row tile leaves nearly all compute units
+        // idle). So does a chunk whose partials the device has no room for.
+        std::unique_lock<std::mutex> partials;
+        if (hyperion::hip::attention_chunk_splits(a)) {
+            hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+            HYP_HIP_CHECK(hipStreamIsCapturing(s, &st));
+            void* own = nullptr;
+            const size_t bytes = hyperion::hip::attention_chunk_workspace_bytes(c.num_kv_heads, c.head_dim);
+            if (st == hipStreamCaptureStatusNone) {
+                partials = std::unique_lock<std::mutex>(stream->attn_mutex);
+                own = attn_partials(*stream, bytes);
+            }
+            if (own != nullptr) {
+                a.workspace = own;
+                a.workspace_bytes = bytes;
+            } else if (static_cast<uint64_t>(L) * (n_heads / c.num_kv_heads) > 64u) {
+                a.workspace = nullptr;
+                a.workspace_bytes = 0;
+            }
+        }
         hyperion::hip::launch_attention(a, s);
     });
 }

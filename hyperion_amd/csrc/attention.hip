@@ -649,8 +649,8 @@ void launch_decode_d(const AttnParams& p, bool prep, hipStream_t stream) {
 namespace {
 
 // Rows of fp32 partials (m, l and head_dim values each) a split workspace holds: every split
-// of the decode form's 16 rows per kv head, or one row tile per compute unit of the chunk form (256 on MI355X; a
-// plan needs no device).
+// of the decode form's 16 rows per kv head, or one row tile per compute unit of the chunk form
+// (256 on MI355X; a plan needs no device).
 size_t workspace_rows(uint32_t n_kv_heads) {
     constexpr size_t kDecodeRows = 16, kPlanComputeUnits = 256;
     return std::max(kAttnMaxSplits * kDecodeRows * n_kv_heads, kPlanComputeUnits * kChunkRows);
@@ -664,20 +664,41 @@ size_t row_bytes(uint32_t head_dim) { return static_cast<size_t>(head_dim) * 4u 
 // (head_dim 512, one kv head) 203 tokens behind 3000 203 -> 57 us, 64 behind 4000 251 -> 56,
 // 1000 behind 3000 250 -> 166; sliding (256, 8 kv heads) 203 behind 700 39 -> 29, 1000
 // behind 700 50 -> 43; half as many splits as the rule gives 73-81 us on the first two.
-uint32_t chunk_splits(uint32_t L, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t keys) {
+uint32_t chunk_splits(uint32_t L, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t keys,
+                      size_t workspace_bytes) {
     const uint32_t G = n_heads / n_kv_heads;
     const uint64_t tiles = (static_cast<uint64_t>(L) * G + kChunkRows - 1u) / kChunkRows * n_kv_heads;
     const uint64_t slots = static_cast<uint64_t>(device_compute_units()) * (head_dim >= 512u ? 1u : 2u);
     const uint64_t blocks = (keys + kKeyBlock - 1u) / kKeyBlock;
-    const uint64_t fit = workspace_rows(n_kv_heads) / (static_cast<uint64_t>(L) * n_heads);
+    const uint64_t fit = workspace_bytes / row_bytes(head_dim) / (static_cast<uint64_t>(L) * n_heads);
     const uint64_t s = std::min({slots / tiles, blocks / 4u, fit, static_cast<uint64_t>(kAttnMaxSplits)});
     return static_cast<uint32_t>(std::max<uint64_t>(s, 1u));
+}
+
+bool decode_form(const AttnArgs& a) { return static_cast<uint64_t>(a.L) * (a.n_heads / a.n_kv_heads) <= 16u; }
+
+// Keys that a row tile of the call sees at most (a window shows it its own tokens' keys and a
+// window before them; the decode form splits all of them).
+uint32_t keys_seen(const AttnArgs& a) {
+    const uint32_t T = a.prefix_len + a.L;
+    if (decode_form(a) || a.window == 0u) return T;
+    const uint32_t G = a.n_heads / a.n_kv_heads;
+    return static_cast<uint32_t>(std::min<uint64_t>(T, uint64_t{a.window} + (kChunkRows + G - 1u) / G));
 }
 
 }  // namespace
 
 size_t attention_workspace_bytes(uint32_t n_kv_heads, uint32_t head_dim) {
     return workspace_rows(n_kv_heads) * row_bytes(head_dim);
+}
+
+size_t attention_chunk_workspace_bytes(uint32_t n_kv_heads, uint32_t head_dim) {
+    return workspace_rows(n_kv_heads) * row_bytes(head_dim);
+}
+
+bool attention_chunk_splits(const AttnArgs& a) {
+    return !decode_form(a) && chunk_splits(a.L, a.n_heads, a.n_kv_heads, a.head_dim, keys_seen(a),
+                                           attention_chunk_workspace_bytes(a.n_kv_heads, a.head_dim)) > 1u;
 }
 
 void launch_kv_write(const uint16_t* k, const uint16_t* v, uint16_t* ck, uint16_t* cv, uint32_t n, uint32_t pos0,
@@ -711,9 +732,10 @@ uint32_t decode_splits(uint32_t n_kv_heads, uint32_t keys) {
     return std::max(1u, std::min(kAttnMaxSplits, (keys + kKeyBlock - 1u) / kKeyBlock));
 }
 
-uint32_t attention_splits(uint32_t L, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t keys) {
+uint32_t attention_splits(uint32_t L, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t keys,
+                          size_t workspace_bytes) {
     if (static_cast<uint64_t>(L) * (n_heads / n_kv_heads) <= 16u) return decode_splits(n_kv_heads, keys);
-    return chunk_splits(L, n_heads, n_kv_heads, head_dim, keys);
+    return chunk_splits(L, n_heads, n_kv_heads, head_dim, keys, workspace_bytes);
 }
 
 void launch_attention(const AttnArgs& a, hipStream_t stream) {
@@ -734,17 +756,15 @@ void launch_attention(const AttnArgs& a, hipStream_t stream) {
     p.window = a.window;
     const uint32_t T = a.prefix_len + a.L;
     p.pos = a.pos;
-    const bool decode = static_cast<uint64_t>(a.L) * p.G <= 16u;
+    const bool decode = decode_form(a);
     if (a.pos != nullptr) {
         // A grid fixed for every position the captured launch will see (the kernel
-        // derives its key ranges from *pos; splits past the keys write empty partials).
+        // derives its key ranges from *pos; splits past the keys write nothing, and the merge
+        // does not read them).
         p.splits = std::max(1u, std::min(a.fixed_splits, kAttnMaxSplits));
         p.keys_per_split = kKeyBlock;
     } else {
-        // (a window shows a row tile at most its own tokens' keys and a window before them)
-        const uint32_t tile_tokens = (kChunkRows + p.G - 1u) / p.G;
-        const uint32_t seen = decode || a.window == 0u ? T : std::min<uint64_t>(T, uint64_t{a.window} + tile_tokens);
-        p.splits = attention_splits(a.L, a.n_heads, a.n_kv_heads, a.head_dim, seen);
+        p.splits = attention_splits(a.L, a.n_heads, a.n_kv_heads, a.head_dim, keys_seen(a), a.workspace_bytes);
         p.keys_per_split = ((T + p.splits - 1u) / p.splits + kKeyBlock - 1u) / kKeyBlock * kKeyBlock;
         if (decode) p.splits = std::max(1u, (T + p.keys_per_split - 1u) / p.keys_per_split);   // no empty split
     }

@@ -482,7 +482,7 @@ void Decoder::forward_chunk(DecoderState& st, const uint32_t* d_ids, uint32_t L,
             // Splits sized for the longest key range the replays can see.
             const uint32_t max_keys = sliding ? std::min(g.window, g.max_positions) + L : g.max_positions;
             aa.pos = d_pos;
-            aa.fixed_splits = hip::attention_splits(L, g.heads, kvh, D, max_keys);
+            aa.fixed_splits = hip::attention_splits(L, g.heads, kvh, D, max_keys, aa.workspace_bytes);
         }
         if (fold_prepare) aa.prep = &pa;
         hip::launch_attention(aa, s);

@@ -150,8 +150,9 @@ void launch_sample_stochastic(const uint16_t* logits, uint32_t vocab, void* work
                               HypTopKSample* out, hipStream_t stream);
 
 // Attention (forward.cc:376-508) over a KV cache prefix and the current chunk; see
-// attention.hip. Calls that leave compute units idle split the keys; the partial sums need
-// attention_workspace_bytes.
+// attention.hip. Calls that leave compute units idle split the keys, and their partial sums go
+// to `workspace`: the decode form (at most 16 query rows per kv head) needs
+// attention_workspace_bytes, the chunk form splits as far as workspace_bytes holds it.
 constexpr uint32_t kAttnMaxSplits = 256;
 struct AttnPrepareArgs;
 struct AttnArgs {
@@ -176,7 +177,13 @@ struct AttnArgs {
     const AttnPrepareArgs* prep = nullptr;
 };
 size_t attention_workspace_bytes(uint32_t n_kv_heads, uint32_t head_dim);
-uint32_t attention_splits(uint32_t L, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t keys);
+// The most that the chunk form splits into, and whether this call (of the chunk form) would
+// split with that much.
+size_t attention_chunk_workspace_bytes(uint32_t n_kv_heads, uint32_t head_dim);
+bool attention_chunk_splits(const AttnArgs& a);
+// Splits of a call whose rows see up to `keys` keys, with that workspace.
+uint32_t attention_splits(uint32_t L, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t keys,
+                          size_t workspace_bytes);
 // Whether AttnArgs::prep can fold the prepare for this geometry: one token runs the decode
 // form (G <= 16 query rows per kv head) and the G query rows and the new K and V of one kv
 // head fit one wave as 64-value units ((G + 2) * head_dim / 64 <= 64).

@@ -319,9 +319,11 @@ HypStatus hyp_sample_greedy_topk(const void* logits, uint32_t rows, uint32_t voc
  * position p in slot p % capacity. A sliding layer's ring (LocalKvCache) is a cache of at
  * least its window; a global layer's cache (GlobalKvCache) is given the context length as
  * capacity - the reference grows it in 256-token steps, which 288 GB of HBM does not need.
- * The handle also owns the workspace of attention's split keys (fixed size: 32768 rows, or
- * 4096 per KV head, of head_dim + 2 fp32 values), so attention on a capturing stream
- * allocates nothing. head_dim: 64, 128, 256 or 512. */
+ * The handle also owns the workspace of decode attention's split keys (at most 16 query rows
+ * per KV head; fixed size: 32768 rows, or 4096 per KV head, of head_dim + 2 fp32 values), so
+ * attention on a capturing stream allocates nothing: calls of that form on one cache that
+ * overlap (on two streams without ordering between them) race. head_dim: 64, 128, 256 or
+ * 512. */
 typedef struct HypKvCacheOpaque* HypKvCache;   /* magic "HPKV" */
 HypStatus hyp_kv_cache_create(uint32_t capacity, uint32_t num_kv_heads, uint32_t head_dim, HypKvCache* out_cache);
 HypStatus hyp_kv_cache_free(HypKvCache* cache);
@@ -343,7 +345,11 @@ HypStatus hyp_kv_cache_write(HypKvCache cache, const void* k, const void* v, uin
  * [offset, offset + L): call it before hyp_kv_cache_write of the chunk, so a ring's prefix
  * is read before the chunk overwrites its slots. prefix_len <= offset and <= capacity (a
  * sliding layer passes min(window, offset), a global one offset). fp32 scores and softmax,
- * P rounded to bf16 for the P.V products, output rounded to bf16. */
+ * P rounded to bf16 for the P.V products, output rounded to bf16. With more than 16 query rows
+ * per KV head a call that splits its keys does so in partials that `stream` owns (32768 rows, or
+ * 4096 per KV head, of head_dim + 2 fp32 values; made by the first such call, freed with the
+ * stream), and such calls may overlap on one cache. Recorded into a graph they use none, and
+ * those of 17 to 64 query rows per KV head the handle's workspace. */
 HypStatus hyp_attention(const void* q, const void* k, const void* v, uint32_t L, uint32_t n_heads, HypKvCache cache,
                         uint32_t offset, uint32_t prefix_len, uint32_t window, void* out, HypStream stream);
 

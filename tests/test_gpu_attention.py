@@ -184,6 +184,73 @@ def test_chunk_dominant_key_precision(stream, place):
     cache.close()
 
 
+def test_chunks_overlap_on_one_cache(stream):
+    """Chunks that split their keys, on two streams over one cache at once (both only read it):
+    each gives the bits of the call alone. 4 tokens (64 query rows per kv head), then 150."""
+    H, KVH, D, prefix, cap = 16, 1, 512, 3000, 3200
+    rng = np.random.default_rng(77)
+    b = lambda scale, *shape: syn.bf16_bits((rng.standard_normal(shape) * scale).astype(np.float32))  # noqa: E731
+    cache = hy.KvCache(cap, KVH, D)
+    _fill_cache(cache, b(1.0, cap, KVH, D), b(1.0, cap, KVH, D), stream)
+    streams = [hy.Stream(), hy.Stream()]
+    for L in (4, 150):
+        say(f"overlapping chunks L={L}")
+        qs = [dev(b(0.1, L, H, D), stream) for _ in streams]
+        outs = [[hy.DeviceArray((L, H, D), np.uint16) for _ in range(6)] for _ in streams]
+        stream.synchronize()
+        call = lambda i, out: hy.call("hyp_attention", qs[i].ptr, None, None, L, H, cache.handle, prefix, prefix,  # noqa: E731
+                                      0, out.ptr, streams[i].handle)
+        alone = []
+        for i, s in enumerate(streams):
+            call(i, outs[i][0])
+            s.synchronize()
+            alone.append(outs[i][0].to_host(s))
+        for n in range(6):
+            for i in range(2):
+                call(i, outs[i][n])
+        for i, s in enumerate(streams):
+            for n in range(6):
+                np.testing.assert_array_equal(outs[i][n].to_host(s), alone[i], err_msg=f"L={L} stream {i} call {n}")
+        for a in (*qs, *outs[0], *outs[1]):
+            a.close()
+    for s in streams:
+        s.synchronize()
+        s.close()
+    cache.close()
+
+
+@pytest.mark.parametrize("L", [4, 150])
+def test_chunk_recorded_into_a_graph(stream, L):
+    """A chunk that splits its keys outside a capture, recorded: in the handle's workspace (64
+    query rows per kv head) or unsplit. Every replay, with eager work between, meets the bar."""
+    H, KVH, D, prefix, cap = 16, 1, 512, 1200, 1400
+    rng = np.random.default_rng(L)
+    b = lambda scale, *shape: syn.bf16_bits((rng.standard_normal(shape) * scale).astype(np.float32))  # noqa: E731
+    q, k, v = b(0.1, L, H, D), b(1.0, L, KVH, D), b(1.0, L, KVH, D)
+    ck, cv = b(1.0, cap, KVH, D), b(1.0, cap, KVH, D)
+    ref = O.attention_f64(q, k, v, ck, cv, prefix, prefix, 0)
+    ck[prefix:prefix + L], cv[prefix:prefix + L] = k, v
+    cache = hy.KvCache(cap, KVH, D)
+    _fill_cache(cache, ck, cv, stream)
+    qd, out, other = dev(q, stream), hy.DeviceArray((L, H, D), np.uint16), hy.DeviceArray((L, H, D), np.uint16)
+    call = lambda o: hy.call("hyp_attention", qd.ptr, None, None, L, H, cache.handle, prefix, prefix, 0, o.ptr,  # noqa: E731
+                             stream.handle)
+    call(other)
+    stream.synchronize()
+    with hy.Graph.capture(stream) as graph:
+        call(out)
+    for rep in range(3):
+        call(other)
+        stream.synchronize()
+        out.upload(np.zeros((L, H, D), np.uint16), stream)
+        graph.launch(stream)
+        _check(out.to_host(stream), ref, np.concatenate([v.reshape(-1), cv.reshape(-1)]), f"L={L} replay {rep}")
+    graph.close()
+    for a in (qd, out, other):
+        a.close()
+    cache.close()
+
+
 def test_kv_cache_write_slots_and_ring_overwrite(stream):
     """Tokens land in slot p % capacity; a write longer than the ring keeps its last
     `capacity` tokens; attention over the written prefix equals attention over the same
