@@ -145,7 +145,7 @@ struct HypKvCacheOpaque {
     uint32_t head_dim = 0;
     DeviceBuffer k;
     DeviceBuffer v;
-    DeviceBuffer workspace;   // decode attention's split partials
+    DeviceBuffer workspace;   // split partials of decode attention, and of small recorded chunks
 };
 
 struct HypGraphOpaque {
@@ -725,7 +725,7 @@ HypStatus hyp_kv_cache_create(uint32_t capacity, uint32_t num_kv_heads, uint32_t
         c->head_dim = head_dim;
         c->k = DeviceBuffer(bytes);
         c->v = DeviceBuffer(bytes);
-        c->workspace = DeviceBuffer(hyperion::hip::attention_workspace_bytes(num_kv_heads, head_dim));
+        c->workspace = DeviceBuffer(hyperion::hip::attention_workspace_bytes(num_kv_heads, head_dim, capacity));
         c->magic = kKvCacheMagic;
         *out_cache = c.release();
     });

@@ -648,14 +648,7 @@ void launch_decode_d(const AttnParams& p, bool prep, hipStream_t stream) {
 
 namespace {
 
-// Rows of fp32 partials (m, l and head_dim values each) a split workspace holds: every split
-// of the decode form's 16 rows per kv head, or one row tile per compute unit of the chunk form
-// (256 on MI355X; a plan needs no device).
-size_t workspace_rows(uint32_t n_kv_heads) {
-    constexpr size_t kDecodeRows = 16, kPlanComputeUnits = 256;
-    return std::max(kAttnMaxSplits * kDecodeRows * n_kv_heads, kPlanComputeUnits * kChunkRows);
-}
-
+// Bytes of one row of fp32 partials (m, l and head_dim values).
 size_t row_bytes(uint32_t head_dim) { return static_cast<size_t>(head_dim) * 4u + 8u; }
 
 // Key splits of the chunk form: as many as the idle compute units take (one workgroup each at
@@ -688,12 +681,17 @@ uint32_t keys_seen(const AttnArgs& a) {
 
 }  // namespace
 
-size_t attention_workspace_bytes(uint32_t n_kv_heads, uint32_t head_dim) {
-    return workspace_rows(n_kv_heads) * row_bytes(head_dim);
+// The decode form: 16 rows per kv head of every split (one per key block, at most
+// kAttnMaxSplits). A chunk of 64 rows has at most a quarter as many splits.
+size_t attention_workspace_bytes(uint32_t n_kv_heads, uint32_t head_dim, uint32_t capacity) {
+    const uint64_t blocks = (uint64_t{capacity} + 64u + kKeyBlock - 1u) / kKeyBlock;
+    return 16u * std::min<uint64_t>(blocks, kAttnMaxSplits) * n_kv_heads * row_bytes(head_dim);
 }
 
+// The chunk form: one row tile per compute unit (256 on MI355X; a plan needs no device), or
+// the decode form's rows of many kv heads.
 size_t attention_chunk_workspace_bytes(uint32_t n_kv_heads, uint32_t head_dim) {
-    return workspace_rows(n_kv_heads) * row_bytes(head_dim);
+    return std::max<size_t>(256u * kChunkRows, size_t{16u} * kAttnMaxSplits * n_kv_heads) * row_bytes(head_dim);
 }
 
 bool attention_chunk_splits(const AttnArgs& a) {

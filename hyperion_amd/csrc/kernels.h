@@ -176,7 +176,8 @@ struct AttnArgs {
     // new token's K/V written to its cache slot by the wave whose keys hold it.
     const AttnPrepareArgs* prep = nullptr;
 };
-size_t attention_workspace_bytes(uint32_t n_kv_heads, uint32_t head_dim);
+// (and holds any chunk of up to 64 query rows per kv head behind a cache of `capacity` tokens).
+size_t attention_workspace_bytes(uint32_t n_kv_heads, uint32_t head_dim, uint32_t capacity);
 // The most that the chunk form splits into, and whether this call (of the chunk form) would
 // split with that much.
 size_t attention_chunk_workspace_bytes(uint32_t n_kv_heads, uint32_t head_dim);

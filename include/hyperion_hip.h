@@ -320,10 +320,10 @@ HypStatus hyp_sample_greedy_topk(const void* logits, uint32_t rows, uint32_t voc
  * least its window; a global layer's cache (GlobalKvCache) is given the context length as
  * capacity - the reference grows it in 256-token steps, which 288 GB of HBM does not need.
  * The handle also owns the workspace of decode attention's split keys (at most 16 query rows
- * per KV head; fixed size: 32768 rows, or 4096 per KV head, of head_dim + 2 fp32 values), so
- * attention on a capturing stream allocates nothing: calls of that form on one cache that
- * overlap (on two streams without ordering between them) race. head_dim: 64, 128, 256 or
- * 512. */
+ * per KV head; fixed size: per KV head 16 rows of head_dim + 2 fp32 values for every 32 tokens
+ * of capacity + 64, at most 4096 rows), so attention on a capturing stream allocates nothing:
+ * calls of that form on one cache that overlap (on two streams without ordering between them)
+ * race. head_dim: 64, 128, 256 or 512. */
 typedef struct HypKvCacheOpaque* HypKvCache;   /* magic "HPKV" */
 HypStatus hyp_kv_cache_create(uint32_t capacity, uint32_t num_kv_heads, uint32_t head_dim, HypKvCache* out_cache);
 HypStatus hyp_kv_cache_free(HypKvCache* cache);

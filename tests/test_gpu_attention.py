@@ -251,6 +251,47 @@ def test_chunk_recorded_into_a_graph(stream, L):
     cache.close()
 
 
+def _free_bytes():
+    hip = ctypes.CDLL("libamdhip64.so")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_cache_handle_memory_follows_its_capacity(stream):
+    """A cache handle holds its K and V and a split workspace for its capacity: 64 caches of 256
+    tokens (0.5 MiB of K and V and 0.3 MiB of workspace each) in 192 MiB, allocation granules
+    included; one of 20000 tokens in its K and V and at most 4096 rows."""
+    stream.synchronize()
+    for cap, count, bound in ((256, 64, 192 << 20), (20000, 4, 4 * (2 * 20000 * 1024 + 4096 * 2056 + (8 << 20)))):
+        before = _free_bytes()
+        caches = [hy.KvCache(cap, 1, 512) for _ in range(count)]
+        used = before - _free_bytes()
+        say(f"{count} caches of {cap} tokens: {used / 2**20:.1f} MiB")
+        assert used <= bound
+        for c in caches:
+            c.close()
+
+
+def test_decode_form_fills_its_workspace(stream):
+    """The most rows and splits that a small cache's workspace has to hold: 16 tokens of one
+    head beside a full prefix, for capacities around a key block."""
+    for cap in (1, 15, 16, 17, 48, 49):
+        say(f"decode form, full cache of {cap}")
+        rng = np.random.default_rng(cap)
+        b = lambda scale, *shape: syn.bf16_bits((rng.standard_normal(shape) * scale).astype(np.float32))  # noqa: E731
+        q, k, v, ck, cv = b(0.3, 16, 2, 64), b(1.0, 16, 2, 64), b(1.0, 16, 2, 64), b(1.0, cap, 2, 64), b(1.0, cap, 2, 64)
+        cache = hy.KvCache(cap, 2, 64)
+        _fill_cache(cache, ck, cv, stream)
+        qd, kd, vd, out = dev(q, stream), dev(k, stream), dev(v, stream), hy.DeviceArray((16, 2, 64), np.uint16)
+        hy.attention(qd, kd, vd, 16, 2, cache, cap, cap, 0, out, stream)
+        ref = O.attention_f64(q, k, v, ck, cv, cap, cap, 0)
+        _check(out.to_host(stream), ref, np.concatenate([v.reshape(-1), cv.reshape(-1)]), f"cap={cap}")
+        for a in (qd, kd, vd, out):
+            a.close()
+        cache.close()
+
+
 def test_kv_cache_write_slots_and_ring_overwrite(stream):
     """Tokens land in slot p % capacity; a write longer than the ring keeps its last
     `capacity` tokens; attention over the written prefix equals attention over the same
