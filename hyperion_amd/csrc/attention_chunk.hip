@@ -41,6 +41,7 @@
 // 1110 -> 364 us (186 -> 566 TFLOP/s); 1000 behind 700 at head_dim 256 (8 kv heads, window 1024)
 // 118 -> 44 us. Without the reads ahead of use a third slower.
 #include "attention.h"
+#include "attention_plan.h"
 #include "common.h"
 #include "kernels.h"
 
@@ -143,8 +144,8 @@ __global__ __launch_bounds__(kThreads, D >= 512u ? 1 : 2) void attn_chunk_kernel
     if (p.window != 0u && p.prefix + t_lo + 1u > p.window) j_lo = p.prefix + t_lo + 1u - p.window;
     const uint32_t j_end = p.prefix + t_hi + 1u;
     const uint32_t blocks = (j_end - j_lo + kKeyBlock - 1u) / kKeyBlock;
-    const uint32_t b0 = blocks * split / p.splits;
-    const uint32_t b1 = blocks * (split + 1u) / p.splits;
+    const uint32_t b0 = split_first_block(blocks, split, p.splits);
+    const uint32_t b1 = split_first_block(blocks, split + 1u, p.splits);
 
     // This wave's rows: their tokens' range, and this lane's last visible key.
     const uint32_t wrow0 = row0 + wave * kWaveRows;
