@@ -114,6 +114,72 @@ __device__ __forceinline__ bf16x8_t round_p(const float* p) {
                                                    cvt_pk_bf16(p[4], p[5]), cvt_pk_bf16(p[6], p[7])));
 }
 
+// One query row again, over its visible keys [j0, j1) of this split alone, against the same
+// reference: the matrix products take masked keys with a probability of 0, which a value of V
+// that is not finite turns into NaN (and the two terms of a probability make NaN of an
+// infinity). Four keys at a time, one per 16 lanes, the next four in flight; fp32 throughout.
+// The sums stay unnormalised, dims 64 c + 4 (lane % 16) + e of o[c][e], in every lane. Rare and
+// slow: 2048 tokens behind 2048 at head_dim 512 with one such value 18 ms.
+template <uint32_t D>
+__device__ __forceinline__ void row_alone(const AttnParams& p, uint32_t hk, size_t orow, uint32_t j0, uint32_t j1,
+                                          float ref, uint32_t lane, float (&o)[D / 64u][4]) {
+    constexpr uint32_t kC = D / 64u;
+    const uint32_t at = (lane & 15u) * 4u;
+    const uint16_t *ck = p.ck, *cv = p.cv, *pk = p.k, *pv = p.v;   // (selected by value, not through memory)
+    const auto load = [&](const uint16_t* row, uint2 (&raw)[kC]) {
+#pragma unroll
+        for (uint32_t c = 0; c < kC; ++c) raw[c] = *reinterpret_cast<const uint2*>(row + 64u * c + at);
+    };
+    const auto value = [](const uint2& w, int e) {
+        const uint32_t two = e < 2 ? w.x : w.y;
+        return (e & 1) != 0 ? __uint_as_float(two & 0xFFFF0000u) : bf16_bits_to_f32(two & 0xFFFFu);
+    };
+    const auto load_keys = [&](uint32_t jb, uint2 (&k)[kC], uint2 (&v)[kC]) {
+        const uint32_t j = min(jb + (lane >> 4), j1 - 1u);
+        const bool cached = pk == nullptr || j < p.prefix;
+        const size_t row = (static_cast<size_t>(cached ? (p.offset - p.prefix + j) % p.cap : j - p.prefix) * p.KVH + hk) * D;
+        load((cached ? ck : pk) + row, k);
+        load((cached ? cv : pv) + row, v);
+    };
+    uint2 q[kC], k[kC], v[kC];
+    load(p.q + orow * D, q);
+#pragma unroll
+    for (uint32_t c = 0; c < kC; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[c][e] = 0.0f;
+    if (j0 < j1) load_keys(j0, k, v);
+    for (uint32_t jb = j0; jb < j1; jb += 4u) {
+        uint2 k_next[kC], v_next[kC];
+        load_keys(jb + 4u, k_next, v_next);   // (past the end: the last key again)
+        float s = 0.0f;
+#pragma unroll
+        for (uint32_t c = 0; c < kC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s = fmaf(value(q[c], e), value(k[c], e), s);
+#pragma unroll
+        for (int d = 1; d < 16; d *= 2) s += __shfl_xor(s, d);
+        if (jb + (lane >> 4) < j1) {
+            const float w = s == s ? __builtin_amdgcn_exp2f(fmaf(s, kLog2e, -ref)) : 0.0f;   // (a NaN score weighs 0)
+#pragma unroll
+            for (uint32_t c = 0; c < kC; ++c)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[c][e] = fmaf(w, value(v[c], e), o[c][e]);
+        }
+#pragma unroll
+        for (uint32_t c = 0; c < kC; ++c) {
+            k[c] = k_next[c];
+            v[c] = v_next[c];
+        }
+    }
+#pragma unroll
+    for (uint32_t c = 0; c < kC; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            o[c][e] += __shfl_xor(o[c][e], 16);
+            o[c][e] += __shfl_xor(o[c][e], 32);
+        }
+}
+
 template <uint32_t D, bool WIDE>
 __global__ __launch_bounds__(kThreads, D >= 512u ? 1 : 2) void attn_chunk_kernel(AttnParams p) {
     resolve_position(p);
@@ -373,45 +439,82 @@ __global__ __launch_bounds__(kThreads, D >= 512u ? 1 : 2) void attn_chunk_kernel
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last loads: none writes LDS past here
     l = half_sum(l);
 
-    // o[dt][i] is dim 32 dt + 8 (i / 4) + 4 h + i % 4 of row n.
-    if (p.splits > 1u) {
-        if (wrow0 + n >= rows) return;
-        const size_t prow = static_cast<size_t>(split) * p.L * p.H + orow;
-#pragma unroll
-        for (uint32_t dt = 0; dt < kDTiles; ++dt)
-#pragma unroll
-            for (uint32_t u = 0; u < 4u; ++u)
-                *reinterpret_cast<float4*>(p.part_o + prow * D + 32u * dt + 8u * u + 4u * h) =
-                    make_float4(o[dt][4 * u], o[dt][4 * u + 1], o[dt][4 * u + 2], o[dt][4 * u + 3]);
-        if (h == 0u) {
-            p.part_ml[prow * 2u] = m;
-            p.part_ml[prow * 2u + 1u] = l;
-        }
-        return;
-    }
-    // The wave's rows through LDS (its own part of the stages, once every wave has left them),
-    // then out as 16-byte pieces of whole rows.
-    __syncthreads();
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    const uint32_t out_lds = lds + wave * kWaveRows * Lds::kOutRow;
+    // Rows with a value that is not finite are formed again, by themselves (row_alone), once they
+    // are out.
+    float zero = 0.0f;
 #pragma unroll
     for (uint32_t dt = 0; dt < kDTiles; ++dt)
 #pragma unroll
-        for (uint32_t u = 0; u < 4u; ++u) {
-            u32x2_t w;
-            w.x = cvt_pk_bf16(o[dt][4 * u] * inv, o[dt][4 * u + 1] * inv);
-            w.y = cvt_pk_bf16(o[dt][4 * u + 2] * inv, o[dt][4 * u + 3] * inv);
-            *reinterpret_cast<HYP_LDS u32x2_t*>(out_lds + n * Lds::kOutRow + (32u * dt + 8u * u + 4u * h) * 2u) = w;
+        for (int i = 0; i < 16; ++i) zero = fmaf(o[dt][i], 0.0f, zero);
+    const uint64_t odd_lanes = __ballot(zero != 0.0f && wrow0 + n < rows);
+    const uint32_t odd_rows = static_cast<uint32_t>(odd_lanes) | static_cast<uint32_t>(odd_lanes >> 32);
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+
+    // o[dt][i] is dim 32 dt + 8 (i / 4) + 4 h + i % 4 of row n.
+    if (p.splits > 1u) {
+        const size_t prow = static_cast<size_t>(split) * p.L * p.H + orow;
+        if (wrow0 + n < rows) {
+#pragma unroll
+            for (uint32_t dt = 0; dt < kDTiles; ++dt)
+#pragma unroll
+                for (uint32_t u = 0; u < 4u; ++u)
+                    *reinterpret_cast<float4*>(p.part_o + prow * D + 32u * dt + 8u * u + 4u * h) =
+                        make_float4(o[dt][4 * u], o[dt][4 * u + 1], o[dt][4 * u + 2], o[dt][4 * u + 3]);
+            if (h == 0u) {
+                p.part_ml[prow * 2u] = m;
+                p.part_ml[prow * 2u + 1u] = l;
+            }
         }
-    __syncthreads();
-    for (uint32_t c = lane; c < kWaveRows * Lds::kChunks; c += 64u) {
-        const uint32_t r = c / Lds::kChunks;
-        const uint32_t gr = wrow0 + r;
-        if (gr >= rows) break;
-        const uint32_t t = gr / p.G;
-        const size_t dst = (static_cast<size_t>(t) * p.H + hk * p.G + (gr - t * p.G)) * D + (c % Lds::kChunks) * 8u;
-        *reinterpret_cast<u32x4_t*>(p.out + dst) =
-            *reinterpret_cast<const HYP_LDS u32x4_t*>(out_lds + r * Lds::kOutRow + (c % Lds::kChunks) * 16u);
+    } else {
+        // The wave's rows through LDS (its own part of the stages, once every wave has left
+        // them), then out as 16-byte pieces of whole rows.
+        __syncthreads();
+        const uint32_t out_lds = lds + wave * kWaveRows * Lds::kOutRow;
+#pragma unroll
+        for (uint32_t dt = 0; dt < kDTiles; ++dt)
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; ++u) {
+                u32x2_t w;
+                w.x = cvt_pk_bf16(o[dt][4 * u] * inv, o[dt][4 * u + 1] * inv);
+                w.y = cvt_pk_bf16(o[dt][4 * u + 2] * inv, o[dt][4 * u + 3] * inv);
+                *reinterpret_cast<HYP_LDS u32x2_t*>(out_lds + n * Lds::kOutRow + (32u * dt + 8u * u + 4u * h) * 2u) = w;
+            }
+        __syncthreads();
+        for (uint32_t c = lane; c < kWaveRows * Lds::kChunks; c += 64u) {
+            const uint32_t r = c / Lds::kChunks;
+            const uint32_t gr = wrow0 + r;
+            if (gr >= rows) break;
+            const uint32_t t = gr / p.G;
+            const size_t dst = (static_cast<size_t>(t) * p.H + hk * p.G + (gr - t * p.G)) * D + (c % Lds::kChunks) * 8u;
+            *reinterpret_cast<u32x4_t*>(p.out + dst) =
+                *reinterpret_cast<const HYP_LDS u32x4_t*>(out_lds + r * Lds::kOutRow + (c % Lds::kChunks) * 16u);
+        }
+    }
+    if (odd_rows == 0u) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the wave's own stores of these rows are done
+    for (uint32_t todo = odd_rows; todo != 0u; todo &= todo - 1u) {
+        const int r = __builtin_ctz(todo);
+        const uint32_t t = (wrow0 + r) / p.G;
+        const size_t row = static_cast<size_t>(t) * p.H + hk * p.G + (wrow0 + r - t * p.G);
+        const uint32_t last = p.prefix + t;
+        const uint32_t first = p.window != 0u && last + 1u > p.window ? last + 1u - p.window : 0u;
+        const float ref = __shfl(m, r);
+        const float scale = __shfl(inv, r);
+        float a[D / 64u][4];
+        row_alone<D>(p, hk, row, max(first, j_lo + b0 * kKeyBlock), min(last + 1u, j_lo + b1 * kKeyBlock),
+                     ref > -__builtin_huge_valf() ? ref : 0.0f, lane, a);
+        if (lane >= 16u) continue;
+#pragma unroll
+        for (uint32_t c = 0; c < D / 64u; ++c) {
+            const uint32_t dim = 64u * c + 4u * lane;
+            if (p.splits > 1u) {
+                *reinterpret_cast<float4*>(p.part_o + (static_cast<size_t>(split) * p.L * p.H + row) * D + dim) =
+                    make_float4(a[c][0], a[c][1], a[c][2], a[c][3]);
+            } else {
+                *reinterpret_cast<uint2*>(p.out + row * D + dim) = make_uint2(
+                    cvt_pk_bf16(a[c][0] * scale, a[c][1] * scale), cvt_pk_bf16(a[c][2] * scale, a[c][3] * scale));
+            }
+        }
     }
 }
 

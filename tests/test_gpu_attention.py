@@ -292,6 +292,48 @@ def test_decode_form_fills_its_workspace(stream):
         cache.close()
 
 
+@pytest.mark.parametrize("L,H,KVH,D,prefix,window,cached", [
+    (8, 16, 1, 512, 40, 0, True),        # one row tile; 2 tokens a wave
+    (3, 16, 1, 512, 8, 0, False),        # rows past the end repeat the last
+    (5, 16, 1, 512, 650, 0, True),       # key splits
+    (64, 4, 2, 256, 33, 0, True),        # 16 tokens a wave, whole waves before the key
+    (70, 4, 2, 128, 50, 20, True),       # a window's edges in the same waves
+    (40, 2, 2, 64, 16, 16, False),
+])
+def test_chunk_values_that_are_not_finite(stream, L, H, KVH, D, prefix, window, cached):
+    """An infinite or NaN value of V reaches the rows that see its key and no others: V of the
+    last token (which no earlier token sees) and of a key that a window shows the first tokens
+    only. Everything else meets the bar against V without them."""
+    say(f"not finite L={L} KVH={KVH} D={D} prefix={prefix} window={window}")
+    T = prefix + L
+    rng = np.random.default_rng(D + L)
+    b = lambda scale, *shape: syn.bf16_bits((rng.standard_normal(shape) * scale).astype(np.float32))  # noqa: E731
+    q, k, v = b(D ** -0.5, L, H, D), b(1.0, T, KVH, D), b(1.0, T, KVH, D)
+    bad = [(T - 1, 3, 0x7F80), (T - 1, D - 9, 0x7FC0)]
+    if window:
+        bad += [(prefix - window + 3, 17, 0xFF80)]      # visible to tokens 0 .. 2
+    vb = v.copy()
+    for j, d, bits in bad:
+        v[j, :, d], vb[j, :, d] = 0, bits
+    cache = hy.KvCache(T, KVH, D)
+    _fill_cache(cache, k, vb, stream)
+    qd, out = dev(q, stream), hy.DeviceArray((L, H, D), np.uint16)
+    kd, vd = dev(k[prefix:], stream), dev(vb[prefix:], stream)
+    hy.call("hyp_attention", qd.ptr, None if cached else kd.ptr, None if cached else vd.ptr, L, H, cache.handle, prefix,
+            prefix, window, out.ptr, stream.handle)
+    got = out.to_host(stream)
+    ref = O.attention_f64(q, k[prefix:], v[prefix:], k, v, prefix, prefix, window)
+    for j, d, bits in bad:
+        t = np.arange(L)
+        sees = (j <= prefix + t) & ((j > prefix + t - window) if window else True)
+        assert np.all(np.isnan(syn.bf16_to_f32(got[sees, :, d])) if bits == 0x7FC0 else got[sees, :, d] == bits), (j, d)
+        got[sees, :, d] = syn.bf16_bits(ref[sees, :, d].astype(np.float32))   # (leaves the bar to the others)
+    _check(got, ref, v, f"L={L} D={D}")
+    for a in (qd, kd, vd, out):
+        a.close()
+    cache.close()
+
+
 def test_kv_cache_write_slots_and_ring_overwrite(stream):
     """Tokens land in slot p % capacity; a write longer than the ring keeps its last
     `capacity` tokens; attention over the written prefix equals attention over the same
