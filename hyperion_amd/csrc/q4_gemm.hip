@@ -32,6 +32,7 @@
 #include <utility>
 
 #include "common.h"
+#include "gemm_plan.h"
 #include "kernels.h"
 #include "q4_dequant.h"
 #include "q4_layout.h"
@@ -58,7 +59,6 @@ struct GemmSegment {
     uint32_t col_begin;   // first column of this segment in the split-k workspace rows
 };
 
-constexpr uint32_t kMaxGemmSegments = 3;
 
 struct GemmParams {
     GemmSegment seg[kMaxGemmSegments];   // segments past nseg are unused
@@ -613,8 +613,6 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2))) 
 // add up through LDS in wave order, so nothing is left to a second launch. Weights
 // dequantize as in the tile kernels (bf16(scale q + bias)). More than two pairs ahead or 16
 // waves per workgroup measured the same or slower (q/k/v at 16 rows 10.6 -> 11.4 with 4 pairs).
-constexpr uint32_t kFewRows = 64;   // at most
-constexpr uint32_t kFewWaves = 8;
 
 template <int MT, int NT, bool DUAL>
 __global__ __launch_bounds__(64 * kFewWaves) void q4_gemm_few_kernel(GemmParams p) {
@@ -876,35 +874,16 @@ void launch_few_m(const GemmParams& p, uint32_t nt, hipStream_t stream) {
     nt >= 2u ? launch_few_t<MT, 2, false>(p, stream) : launch_few_t<MT, 1, false>(p, stream);
 }
 
-// Whether the few-row kernel takes the call. Its time grows with rows x column tiles (each
-// wave reads its rows of X from L2, about 12 TB/s over the chip), the tile kernels' hardly
-// below 128 rows. Measured, tile kernels against it (us, weights alternating): gate + up
-// [2 x 15360, 3840] 38.8 -> 20.8 at 16 rows, 37.4 -> 27.5 at 32, but 37.5 -> 42.5 at 33; down
-// [3840, 15360] 56.4 -> 11.9 at 5, 18.8 at 16, 31.4 at 32, 45.6 at 48, 58.0 -> 58.6 at 64; q/k/v
-// [8192, 3840] 25.3 -> 8.8 at 16, 27.1 -> 19.5 at 64; o [3840, 4096] 23.5 -> 7.2 at 16, 25.6 ->
-// 18.8 at 64; [15360, 3840] 27.1 -> 16.9 at 32, 28.9 -> 35.2 at 64; [262144, 3840] 323 -> 190 at
-// 32. So: always up to 32 rows, to 64 where the column tiles are at most two per compute unit.
-bool few_rows(const GemmParams& p) {
-    uint64_t tiles = 0;
-    for (uint32_t i = 0; i < p.nseg; ++i) tiles += p.seg[i].row_tiles;
-    return p.m <= 32u || (p.m <= kFewRows && tiles <= 2u * device_compute_units());
+GemmShape shape_of(const GemmParams& p) {
+    GemmShape g{p.m, p.pairs, p.nseg, {}, p.dual != 0u};
+    for (uint32_t i = 0; i < p.nseg; ++i) g.n[i] = p.seg[i].n;
+    return g;
 }
 
 void launch_few(GemmParams p, hipStream_t stream) {
-    // As many column tiles per wave (they share its X reads) as leave 7 waves per compute unit
-    // with every tile's pairs over 8 waves, then the fewest waves per tile that still do; from
-    // 33 rows on at most 2 (registers, and the LDS of the sums). At 16 rows (us): [15360, 3840]
-    // 18.7, 13.2 and 12.0 with 1, 2 and 4 tiles per wave, q/k/v [8192, 3840] 10.9, 8.5 and 11.4,
-    // down [3840, 15360] 19.0, 21.5 and 30.1.
-    const uint64_t cus = device_compute_units();
-    uint64_t tiles = 0;
-    for (uint32_t i = 0; i < p.nseg; ++i) tiles += p.seg[i].row_tiles;
-    const uint32_t nt_max = p.m <= 32u ? 4u : 2u;
-    uint32_t nt = p.dual != 0u ? 2u : 1u;
-    while (nt < nt_max && tiles / (2u * nt) * kFewWaves >= 7u * cus) nt *= 2u;
-    uint32_t s = 1u;
-    while (s < kFewWaves && tiles / nt * s < 7u * cus && 2u * s <= p.pairs) s *= 2u;
-    p.ksplit = s;
+    const FewRowShape f = few_row_shape(shape_of(p), device_compute_units());
+    const uint32_t nt = f.tiles;
+    p.ksplit = f.splits;
     switch ((p.m + 15u) / 16u) {
         case 1: launch_few_m<1>(p, nt, stream); break;
         case 2: launch_few_m<2>(p, nt, stream); break;
@@ -948,20 +927,6 @@ GemmParams group_params(const Q4Matrix* const* ws, uint16_t* const* ys, uint32_t
     return p;
 }
 
-// Bytes of the fixed scratch of launch_q4_gemm_noalloc (below).
-constexpr size_t kNoAllocScratchBytes = size_t{64} << 20;
-
-// The tile kernels.
-enum class GemmKernel : uint32_t {
-    kGroup128 = 1,   // q4_gemm_g_kernel<8, 2, 8>: 128 x 256, group step, one per CU
-    kGroup256 = 2,   // q4_gemm_g_kernel<16, 2, 8>: 256 x 256, group step, one per CU
-};
-
-struct GemmChoice {
-    GemmKernel kernel;
-    uint32_t ksplit;
-};
-
 template <bool DUAL>
 void launch_kernel(GemmParams& p, GemmKernel kernel, hipStream_t stream) {
     switch (kernel) {
@@ -978,75 +943,6 @@ void launch_params(GemmParams& p, GemmKernel kernel, hipStream_t stream) {
         launch_kernel<false>(p, kernel, stream);
     }
     HYP_HIP_CHECK(hipGetLastError());
-}
-
-// Workgroups of one k split: (rows / tile rows) x (column tiles over the segments).
-uint64_t gemm_tiles(const GemmParams& p, uint32_t rows, uint32_t cols) {
-    uint64_t tn = 0;
-    for (uint32_t i = 0; i < p.nseg; ++i) tn += (p.seg[i].n + cols - 1u) / cols;
-    return static_cast<uint64_t>((p.m + rows - 1u) / rows) * tn;
-}
-
-// Smallest split (<= 4, at least 6 pairs in each) whose grid of `tiles` x split reaches
-// 90% of the CUs.
-uint32_t fill_split(const GemmParams& p, uint64_t tiles, uint64_t cus) {
-    uint32_t s = 1u;
-    while (s < 4u && tiles * s * 10u < cus * 9u && (p.pairs + s) / (s + 1u) >= 6u) ++s;
-    return s;
-}
-
-// k splits that fill the compute units, at most 4 (the split count of small launches, and the
-// bound that the fixed scratch of launch_q4_gemm_noalloc is checked against).
-uint32_t filling_split(const GemmParams& p) {
-    const uint64_t cus = device_compute_units();
-    const uint64_t big = gemm_tiles(p, 256u, 256u);
-    if (big * 10u >= cus * 9u) return 1u;
-    if (p.pairs >= 64u) {
-        const uint32_t s = fill_split(p, big, cus);
-        if (big * s * 10u >= cus * 9u) return s;
-    }
-    const uint64_t mid = gemm_tiles(p, 128u, 256u);
-    const uint32_t s = fill_split(p, mid, cus);
-    if (mid * s * 10u >= cus * 6u) return s;
-    return fill_split(p, gemm_tiles(p, 128u, 128u), cus);
-}
-
-// Kernel and split per call: the ones with the least estimated time,
-//   4 us + rounds of one workgroup per compute unit x groups per split x time per group
-//   + (split) 4 us + the partials' write and read at 5.5 TB/s,
-// where a group (64 k) of the 128-row kernel takes 0.72 us, of the 256-row kernel 1.3 us, and
-// up to 0.95 and 1.65 us as the grid covers the compute units. From a sweep of the projections
-// at 100 to 2048 rows, all splits to 12, which the estimate meets within about 10%: the ragged
-// grids are what it is for, where filling the compute units by splitting runs into a second
-// round. Against that rule (us): down [3840, 15360] 203 rows 61.8 -> 43.8, 700 rows 148.6 ->
-// 111.6, 1111 rows 194 -> 160; q/k/v [8192, 3840] 300 rows 56.0 -> 42.4, 700 rows 77.6 -> 54.4; o
-// [3840, 4096] 700 rows 58.9 -> 43.4; [15360, 3840] 300 rows 74.1 -> 54.0. The 128 x 128
-// pair-step kernel is at best equal to the 128 x 256 one at the same split (two workgroups per
-// compute unit, each waiting for its loads), and kept for narrow outputs of at most 128 columns.
-GemmChoice choose_gemm(const GemmParams& p) {
-    const uint64_t cus = device_compute_units();
-    const uint32_t most = filling_split(p);
-    GemmChoice best{GemmKernel::kGroup128, 1u};
-    double best_us = 1e30;
-    for (const GemmKernel kernel : {GemmKernel::kGroup256, GemmKernel::kGroup128}) {
-        const bool big = kernel == GemmKernel::kGroup256;
-        const uint64_t tiles = gemm_tiles(p, big ? 256u : 128u, 256u);
-        for (uint32_t s = 1u; s <= 16u && (p.pairs + s - 1u) / s >= 3u; ++s) {
-            const uint64_t bytes = static_cast<uint64_t>(s) * p.m * p.n_total * sizeof(float);
-            if (s > most && bytes > kNoAllocScratchBytes) break;   // larger partials only where filling took them
-            const uint64_t grid = tiles * s;
-            const double cover = std::min(1.0, static_cast<double>(grid) / cus);
-            const double full = std::max(0.0, 2.0 * cover - 1.0);
-            const double group = big ? 1.3 + 0.35 * full : 0.72 + 0.23 * full;
-            double us = 4.0 + static_cast<double>((grid + cus - 1u) / cus) * (2u * ((p.pairs + s - 1u) / s)) * group;
-            if (s > 1u) us += 4.0 + 2.0 * bytes / 5.5e6;
-            if (us < best_us) {
-                best_us = us;
-                best = {kernel, s};
-            }
-        }
-    }
-    return best;
 }
 
 // Where the split-k partials of one call live: a stream-ordered temporary
@@ -1139,8 +1035,9 @@ float* noalloc_scratch() {
 void launch_q4_gemm_group(const Q4Matrix* const* ws, uint16_t* const* ys, uint32_t count, const uint16_t* x,
                           uint32_t m, hipStream_t stream) {
     GemmParams p = group_params(ws, ys, count, x, m);
-    if (few_rows(p)) return launch_few(p, stream);
-    const GemmChoice c = choose_gemm(p);
+    const GemmShape g = shape_of(p);
+    if (few_rows(g, device_compute_units())) return launch_few(p, stream);
+    const GemmChoice c = choose_gemm(g, device_compute_units());
     launch_split(p, c.kernel, c.ksplit, stream);
 }
 
@@ -1150,9 +1047,10 @@ void launch_q4_gemm_gate_up(const Q4Matrix& gate, const Q4Matrix& up, const uint
     const Q4Matrix* ws[2] = {&gate, &up};
     uint16_t* ys[2] = {y, nullptr};
     GemmParams p = group_params(ws, ys, 2u, x, m);
-    const GemmChoice c = choose_gemm(p);   // the kernel and split of the grouped gate/up launch
     p.dual = 1u;
-    if (few_rows(p)) return launch_few(p, stream);
+    const GemmShape g = shape_of(p);
+    if (few_rows(g, device_compute_units())) return launch_few(p, stream);
+    const GemmChoice c = choose_gemm(g, device_compute_units());   // those of the grouped gate/up launch
     launch_split(p, c.kernel, c.ksplit, stream);
 }
 
@@ -1167,11 +1065,12 @@ void launch_q4_gemm_noalloc(const Q4Matrix& w, const uint16_t* x, uint32_t m, ui
     uint16_t* ys[1] = {y};
     GemmParams p = group_params(ws, ys, 1u, x, m);
     // The same kernel and split as launch_q4_gemm.
-    if (few_rows(p)) return launch_few(p, stream);
-    const GemmChoice c = choose_gemm(p);
-    const uint64_t filled = static_cast<uint64_t>(filling_split(p)) * m * p.n_total * sizeof(float);
-    HYP_REQUIRE(filling_split(p) == 1u || filled <= kNoAllocScratchBytes, HYP_STATUS_INVALID_ARGUMENT,
-                "gemm: this call's k splits may need " + std::to_string(filled) +
+    const GemmShape g = shape_of(p);
+    if (few_rows(g, device_compute_units())) return launch_few(p, stream);
+    const GemmChoice c = choose_gemm(g, device_compute_units());
+    const uint32_t filled = filling_split(g, device_compute_units());
+    HYP_REQUIRE(filled == 1u || partial_bytes(g, filled) <= kNoAllocScratchBytes, HYP_STATUS_INVALID_ARGUMENT,
+                "gemm: this call's k splits may need " + std::to_string(partial_bytes(g, filled)) +
                     " bytes of partial sums; the no-allocation scratch holds " + std::to_string(kNoAllocScratchBytes) +
                     " bytes");
     SplitWorkspace wsp;

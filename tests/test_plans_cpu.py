@@ -30,3 +30,23 @@ def test_key_blocks_of_a_split(plans):
     for blocks, splits in cases:
         for s in {0, 1, splits // 2, splits - 1, splits}:
             assert f(blocks, s, splits) == blocks * s // splits, (blocks, s, splits)
+
+
+def gemm(plans, m, ns, k, dual=False, cus=256):
+    """(kernel, splits, tiles per wave) of a call; kernel "few", 128 or 256."""
+    out = (ctypes.c_uint32 * 3)()
+    plans.plan_gemm(m, k, len(ns), (ctypes.c_uint32 * len(ns))(*ns), int(dual), cus, out)
+    return ("few", 128, 256)[out[0]], out[1], out[2]
+
+
+def test_gemm_choice_at_measured_calls(plans):
+    """The choice at calls whose alternatives were measured (us, the choice first): q/k/v at 512
+    rows 49.1 against 50.0 unsplit (54 on weights read from HBM), at 640 rows 53.5 unsplit; down
+    at 2048 rows 208 against 221 unsplit; [3840, 8192] at 700 rows 61.8 against 68.1 (128-row
+    tiles, split 2); gate/up at 512 rows 108 unsplit."""
+    assert gemm(plans, 512, (4096, 2048, 2048), 3840)[:2] == (128, 2)
+    assert gemm(plans, 512, (8192,), 3840)[:2] == (128, 2)
+    assert gemm(plans, 640, (4096, 2048, 2048), 3840)[:2] == (128, 1)
+    assert gemm(plans, 2048, (3840,), 15360)[:2] == (256, 2)
+    assert gemm(plans, 700, (3840,), 8192)[:2] == (256, 5)
+    assert gemm(plans, 512, (15360, 15360), 3840, dual=True)[:2] == (256, 1)
