@@ -202,10 +202,11 @@ HypStatus hyp_qmatmul(HypQWeight weight, const void* x, uint32_t m, void* y, Hyp
  * is the same bits; where hyp_qmatmul's prefill GEMM (m > 4) splits k, the fp32 partial
  * sums go to a fixed 64 MiB device scratch array that the library holds on each device
  * it runs on until the process ends (enough for every projection of a 12B layer at
- * m <= 2048). A call whose partials would exceed it returns INVALID_ARGUMENT and runs
- * nothing. All calls on one device share that scratch: calls that overlap on one device
- * (e.g. on two streams without ordering between them) race; calls on one stream are
- * ordered and safe. Nothing in the scratch needs clearing between calls. */
+ * m <= 2048). A call whose partials, or those of the k splits that would fill the device's
+ * compute units (at most 4), exceed it returns INVALID_ARGUMENT and runs nothing. All calls
+ * on one device share that scratch: calls that overlap on one device (e.g. on two streams
+ * without ordering between them) race; calls on one stream are ordered and safe. Nothing in
+ * the scratch needs clearing between calls. */
 HypStatus hyp_qmatmul_noalloc(HypQWeight weight, const void* x, uint32_t m, void* y, HypStream stream);
 
 /* hyp_qmatmul with an epilogue; HYP_EPILOGUE_SOFTCAP with cap > 0 is the tied

@@ -384,8 +384,8 @@ def test_gemm_prefill_projections_sampled(stream, m):
 @pytest.mark.parametrize("m", [512, 1024, 2048])
 def test_gemm_grouped_qkv_layer_shapes(stream, m):
     """The grouped q/k/v call of a layer at prefill sizes ([4096|2048|2048, 3840] in one
-    launch): m = 512 takes the 128 x 256 group-step kernel with 2 k splits, m = 1024 the
-    same unsplit and m = 2048 the 256 x 256 one. Sampled rows against the fp64 product with
+    launch): m = 512 takes the 128-row tile kernel with 2 k splits, m = 1024 the same unsplit
+    and m = 2048 the 256-row one. Sampled rows against the fp64 product with
     the kernel's bf16 weights, and sig_rel <= 1e-2 against the fp64 truth."""
     k = 3840
     say(f"gemm grouped q/k/v m={m}")
@@ -415,11 +415,11 @@ def test_gemm_exact_integer_and_ragged_tiles(stream):
 
 
 def test_gemm_split_k_grouped_and_exact(stream):
-    """Grids of at most one workgroup per CU split k (fp32 partials summed in order): a
-    grouped call (n = 40, 24, 1000: the reduction maps workspace columns back to three
-    outputs) with an odd group count (k = 4160), against the fp64 product with the
-    kernel's bf16 weights; and exact integer inputs (300 x 200 x 4096, 4 splits of 8
-    pairs), bit-exact."""
+    """Grids short of the CUs split k (fp32 partials summed in order): a grouped call (n = 40,
+    24, 1000: the reduction maps workspace columns back to three outputs) with an odd group
+    count (k = 4160, 11 splits of 3 pairs), against the fp64 product with the kernel's bf16
+    weights; and exact integer inputs (300 x 200 x 4096, 11 splits, the last of 2 pairs),
+    bit-exact."""
     m, k = 200, 4160
     ws = [syn.q4_weights(n, k, seed=1400 + n) for n in (40, 24, 1000)]
     x = syn.activations(m, k, seed=1410)
@@ -448,16 +448,19 @@ FEW_CASES = [
     (32, (15360,), 448),            # four column tiles per wave
     (31, (8200,), 320),             # two, the last wave's second past the end
     (33, (2048, 16), 1088),
-    (48, (4096, 2048, 2041), 256),  # 513 column tiles: the tile kernels again from 33 rows on
+    (48, (4096, 2048, 2041), 256),  # 512 column tiles, the most from 33 rows on
     (64, (3840,), 704),
+    # past the kernel's bounds: 513 column tiles, and 200 MB of X read by the waves
+    (48, (4096, 2048, 2049), 256),
+    (33, (3840,), 15360),
 ]
 
 
 @pytest.mark.parametrize("m,ns,k", FEW_CASES)
 def test_gemm_few_rows_exact(stream, m, ns, k):
-    """The few-row kernel at the edges of its tiles and splits: integer inputs, whose sums are
-    exact in fp32 in any order, so every output equals the exact product rounded once; X rows past m and groups past k must
-    not contribute (the row after the last is NaN)."""
+    """The few-row kernel at the edges of its tiles, splits and bounds: integer inputs, whose sums
+    are exact in fp32 in any order, so every output equals the exact product rounded once; X
+    rows past m and groups past k must not contribute (the row after the last is NaN)."""
     say(f"few rows m={m} ns={ns} k={k}")
     rng = np.random.default_rng(m * 100 + k)
     x = rng.integers(-1, 2, size=(m + 1, k)).astype(np.float32)
@@ -478,11 +481,69 @@ def test_gemm_few_rows_exact(stream, m, ns, k):
         a.close()
 
 
+def test_gemm_few_rows_vocabulary_width(stream):
+    """The few-row kernel at the LM head's [262144, 3840] (0.5 GB of codes), one row tile and two,
+    exact on integers; the weight rows repeat every 4099."""
+    n, k, period = 262144, 3840, 4099
+    say(f"few rows [{n}, {k}]")
+    rng = np.random.default_rng(21)
+    codes = rng.integers(0, 16, size=(period, k)).astype(np.uint8)
+    rows = np.arange(n) % period
+    qw = hy.QWeight.from_host(syn.pack_codes(codes)[rows],
+                              syn.bf16_bits(np.full((1, k // 64), 2.0**-7, np.float32)).repeat(n, 0),
+                              syn.bf16_bits(np.full((1, k // 64), -(2.0**-4), np.float32)).repeat(n, 0))
+    for m in (16, 31):
+        x = rng.integers(-1, 2, size=(m, k)).astype(np.float32)
+        xd, y = dev(syn.bf16_bits(x), stream), hy.DeviceArray((m, n), np.uint16)
+        hy.qmatmul(qw, xd, m, y, stream)
+        exact = (x.astype(np.float64) @ (codes.astype(np.float64) - 8).T) * 2.0**-7
+        np.testing.assert_array_equal(y.to_host(stream), syn.bf16_bits(exact.astype(np.float32))[:, rows], err_msg=f"m={m}")
+        xd.close()
+        y.close()
+    qw.close()
+
+
+TILE_CASES = [
+    # m, widths, k: the tile kernels' forms (kernel and k splits of each in test_plans_cpu.py)
+    (700, (3840,), 15360),       # 256 rows, 5 splits, the last row tile part-empty
+    (1001, (3000, 832), 15424),  # 256 rows, 4 splits, two segments, an odd group count
+    (1001, (3837,), 15424),      # the same with n % 8 != 0: element-wise reduction
+    (2000, (15357,), 3904),      # 256 rows unsplit, element-wise stores, an odd group count
+    (500, (2041, 2048), 8256),   # 128 rows, 4 splits, a segment that starts off 8 columns
+    (700, (2999,), 4160),        # 128 rows, 3 splits
+    (300, (15360,), 3840),       # 128 rows unsplit
+]
+
+
+@pytest.mark.parametrize("m,ns,k", TILE_CASES)
+def test_gemm_tile_forms_exact(stream, m, ns, k):
+    """Both tile kernels, split and unsplit, with ragged rows, widths and group counts: integer
+    inputs, whose sums (below 2^17) are exact in fp32 in any order, on sampled rows and the last
+    row tile."""
+    say(f"tile forms m={m} ns={ns} k={k}")
+    rng = np.random.default_rng(m + k)
+    x = rng.integers(-1, 2, size=(m, k)).astype(np.float32)
+    xd = dev(syn.bf16_bits(x), stream)
+    check = np.unique(np.concatenate([[0], rng.choice(m, 24), np.arange(m - 12, m)]))
+    qws, ys, exact = [], [], []
+    for n in ns:
+        codes = rng.integers(0, 16, size=(n, k)).astype(np.uint8)
+        qws.append(hy.QWeight.from_host(syn.pack_codes(codes), syn.bf16_bits(np.full((n, k // 64), 2.0**-7, np.float32)),
+                                        syn.bf16_bits(np.full((n, k // 64), -(2.0**-4), np.float32))))
+        ys.append(hy.DeviceArray((m, n), np.uint16))
+        exact.append((x[check] @ (codes.astype(np.float32) - 8).T) * 2.0**-7)
+    hy.qmatmul_group(qws, xd, m, ys, stream)
+    for n, y, e in zip(ns, ys, exact):
+        np.testing.assert_array_equal(y.to_host(stream)[check], syn.bf16_bits(e.astype(np.float32)), err_msg=f"n={n}")
+    for a in (*qws, *ys, xd):
+        a.close()
+
+
 @pytest.mark.parametrize("n,k", [(8200, 192), (8195, 320), (8200, 3840)])
 def test_gemm_group_step_tiles(stream, n, k):
-    """Grids of >= 0.9 workgroups per CU in 256 x 256 tiles select the 256-row group-step kernel: ragged m
-    (2000 rows, the last row tile part-empty), n with a part-empty 16-row tile (8200) or
-    n % 8 != 0 (8195: the element-wise store path), odd group counts (k = 192, 320).
+    """The 128-row tile kernel unsplit on grids of two rounds: ragged m (2000 rows, the last row
+    tile part-empty), n with a part-empty 16-column tile (8200) or n % 8 != 0 (8195: the
+    element-wise store path), odd group counts (k = 192, 320).
     Sampled rows against the fp64 product with the kernel's bf16 weights, and all rows
     exact on integer inputs."""
     m = 2000
@@ -506,10 +567,10 @@ def test_gemm_group_step_tiles(stream, n, k):
 
 @pytest.mark.parametrize("m,n,splits", [(1300, 6000, 1), (700, 2999, 4)])
 def test_gemm_group_step_128_rows(stream, m, n, splits):
-    """Mid-size grids select the 128 x 256 group-step kernel, unsplit (11 x 24 tiles) or
-    with 4 k splits (6 x 12 tiles; n = 2999 is odd, so the split sums take the
-    element-wise reduction): ragged m (the last 128-row tile part-empty), n not a multiple
-    of 256, an odd group count (k = 4160: 65 groups, so the last pair is half empty).
+    """The 256-row tile kernel unsplit (6 x 24 tiles) and the 128-row one with 3 k splits (6 x 12
+    tiles; n = 2999 is odd, so the split sums take the element-wise reduction; `splits` was its
+    count when the case was written): ragged m, n not a multiple of 256, an odd group count
+    (k = 4160: 65 groups, so the last pair is half empty).
     Sampled rows against the fp64 product with the kernel's bf16 weights, and exact
     integer inputs on sampled rows including the last row tile."""
     k = 4160
@@ -534,7 +595,7 @@ def test_gemm_group_step_128_rows(stream, m, n, splits):
 @pytest.mark.parametrize("m,n,k", [(2048, 40, 128), (300, 200, 4096)])
 def test_gemm_output_not_16_byte_aligned(stream, m, n, k):
     """y one element past a 16-byte boundary: the 16-byte store paths (the tile epilogue,
-    and the 8-column split-k reduction for the 4-split 300 x 200 x 4096 call) fall back
+    and the 8-column split-k reduction for the split 300 x 200 x 4096 call) fall back
     to element stores; results equal the aligned call's bit for bit."""
     import ctypes
     say(f"gemm unaligned y m={m} n={n} k={k}")
@@ -553,12 +614,11 @@ def test_gemm_output_not_16_byte_aligned(stream, m, n, k):
 
 
 def test_gemm_group_step_split_k(stream):
-    """A long k (129 groups) on a grid short of the CUs (8 x 12 tiles of 256 x 256) runs the
-    256-row group-step kernel with k split 3 ways (22-pair ranges, the last covering 41
-    groups and ending on a half pair): a grouped call over two segments (n = 1000, 2000) with ragged
-    m = 2000, against the fp64 product with the kernel's bf16 weights on sampled rows; and
-    exact integer inputs on one [3000, 8256] matrix, bit-exact on sampled rows including
-    the part-empty last row tile."""
+    """A long k with an odd group count (129) through the 128-row tile kernel unsplit: a grouped
+    call over two segments (n = 1000, 2000) with ragged m = 2000, against the fp64 product with
+    the kernel's bf16 weights on sampled rows; and exact integer inputs on one [3000, 8256]
+    matrix, bit-exact on sampled rows including the part-empty last row tile. (The split forms:
+    test_gemm_tile_forms_exact.)"""
     m, k = 2000, 8256
     say(f"gemm group-step split-k m={m} k={k}")
     ws = [syn.q4_weights(n, k, seed=1500 + n) for n in (1000, 2000)]
@@ -632,9 +692,9 @@ def test_gate_up_gelu_fused(stream, m):
 
 
 DUAL_CASES = [
-    # n, k, m: the 256 x 256 group-step kernel; the 128 x 256 one; the pair-step kernel;
-    # the pair-step kernel split 4 ways (the dual split-k reduce); an odd group count; a
-    # ragged n; the smallest GEMM batch
+    # n, k, m: the 256-row tile kernel twice; the 128-row one with 2 k splits (the dual split-k
+    # reduce); the few-row kernel at 64 rows, with an odd group count, with a ragged n, and at
+    # the smallest GEMM batch
     (15360, 3840, 2048),
     (15360, 3840, 512),
     (15360, 3840, 64),
@@ -642,6 +702,20 @@ DUAL_CASES = [
     (384, 192, 40),
     (1000, 640, 33),
     (15360, 3840, 5),
+    # few rows, four tiles a wave (two gate/up pairs): one row tile and two; the last wave's
+    # second pair past the end (959 and 513 tiles), odd group counts
+    (15360, 3840, 16),
+    (15360, 3840, 17),
+    (15336, 3840, 31),
+    (15360, 3840, 32),
+    (8200, 4160, 32),
+    (8200, 320, 20),
+    # the tile kernels with a ragged n and an odd group count: 128 rows unsplit and split, 256
+    # rows unsplit and split
+    (15355, 704, 600),
+    (3001, 3904, 300),
+    (15357, 3904, 2000),
+    (1917, 15424, 700),
 ]
 
 

@@ -65,3 +65,26 @@ def test_few_row_bounds(plans):
         assert kernel(64, ns, k) == "few" and kernel(65, ns, k) != "few"
     assert kernel(48, (3840,), 8192) == "few" and kernel(56, (3840,), 8192) != "few"
     assert kernel(64, (8192,), 256) == "few" and kernel(64, (8193,), 256) != "few"   # 512 and 513 column tiles
+
+
+def test_gpu_cases_reach_the_kernels_they_name(plans):
+    """The paths of the GEMM cases in test_gpu_parity.py and test_zz_no_alloc.py, case by case: a
+    rule that moves a case to another kernel or split fails here rather than leave a form
+    without a test."""
+    from test_gpu_parity import DUAL_CASES, FEW_CASES, TILE_CASES
+    few = [gemm(plans, *c) for c in FEW_CASES]
+    assert few == [("few", 1, 1), ("few", 2, 1), ("few", 8, 1), ("few", 8, 1), ("few", 4, 4), ("few", 2, 2),
+                   ("few", 8, 1), ("few", 2, 2), ("few", 4, 1), (128, 1, 0), (128, 12, 0)]
+    assert [gemm(plans, m, (262144,), 3840) for m in (16, 31)] == [("few", 1, 4)] * 2
+    assert [gemm(plans, *c)[:2] for c in TILE_CASES] == [(256, 5), (256, 4), (256, 4), (256, 1), (128, 4), (128, 3), (128, 1)]
+    dual = [gemm(plans, m, (n, n), k, dual=True) for n, k, m in DUAL_CASES]
+    assert dual == [(256, 1, 0), (256, 1, 0), (128, 2, 0), ("few", 8, 2), ("few", 2, 2), ("few", 4, 2), ("few", 4, 4),
+                    ("few", 4, 4), ("few", 4, 4), ("few", 4, 4), ("few", 4, 4), ("few", 8, 4), ("few", 2, 4),
+                    (128, 1, 0), (128, 3, 0), (256, 1, 0), (256, 5, 0)]
+    qkv = (4096, 2048, 2048)
+    assert [gemm(plans, m, qkv, 3840)[:2] for m in (512, 1024, 2048)] == [(128, 2), (128, 1), (256, 1)]
+    for m, ns, k, want in ((200, (40, 24, 1000), 4160, (128, 11)), (300, (200,), 4096, (128, 11)),
+                           (2000, (8200,), 192, (128, 1)), (2000, (8195,), 320, (128, 1)), (2000, (8200,), 3840, (128, 1)),
+                           (1300, (6000,), 4160, (256, 1)), (2000, (1000, 2000), 8256, (128, 1)), (2000, (3000,), 8256, (128, 1)),
+                           (2048, (3840,), 15360, (256, 2)), (512, (2048,), 3840, (128, 6)), (1024, (4608,), 65536, (256, 3))):
+        assert gemm(plans, m, ns, k)[:2] == want, (m, ns, k)

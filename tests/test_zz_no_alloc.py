@@ -3,8 +3,8 @@
 Both are called through the C ABI (ctypes). The no-allocation form runs the same kernels
 and k splits, with the split-k partial sums in the library's fixed device scratch, so its
 output must equal hyp_qmatmul's bit for bit. Two calls in a row share the scratch, the
-second with a smaller input; a call whose partials exceed the scratch is refused before
-anything runs; and the entry can be recorded into a graph and replayed.
+second with a smaller input; a call that may need more partials than the scratch holds is
+refused before anything runs; and the entry can be recorded into a graph and replayed.
 """
 import ctypes
 import sys
@@ -46,7 +46,7 @@ def _both(stream, n, k, m, seed):
 
 def test_noalloc_equals_qmatmul_two_calls_second_smaller(stream):
     # down [3840, 15360] at m = 2048: k split 2 ways, 62.9 MB of partials in the scratch;
-    # then k [2048, 3840] at m = 512: split 4 ways, 16.8 MB, over the first call's contents.
+    # then k [2048, 3840] at m = 512: split 6 ways, 25.2 MB, over the first call's contents.
     for n, k, m, seed in ((3840, 15360, 2048, 3000), (2048, 3840, 512, 3010), (15360, 3840, 1, 3020)):
         say(f"noalloc [{n},{k}] m={m}")
         ya, yb, x, wsb = _both(stream, n, k, m, seed)
@@ -57,8 +57,9 @@ def test_noalloc_equals_qmatmul_two_calls_second_smaller(stream):
 
 
 def test_noalloc_refuses_partials_beyond_the_scratch(stream):
-    # [4608, 65536] at m = 1024 splits k 4 ways: 75.5 MB of partials > 64 MiB. The call is
-    # refused and leaves y untouched; hyp_qmatmul (which allocates) still runs it.
+    # [4608, 65536] at m = 1024: filling the compute units takes 4 k splits and 75.5 MB of
+    # partials > 64 MiB, by which the call is refused (the 3 splits it would run with, 56.6 MB,
+    # have no say). It leaves y untouched; hyp_qmatmul (which allocates) runs it.
     n, k, m = 4608, 65536, 1024
     say(f"noalloc oversize [{n},{k}] m={m}")
     qw = hy.QWeight.from_host(*syn.q4_weights(n, k, seed=3030))
