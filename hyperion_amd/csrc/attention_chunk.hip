@@ -24,16 +24,18 @@
 //    probability is then no longer the exact 1 of a running maximum: rounded to bf16 against an
 //    unrounded denominator it would leave a row that one key dominates an error of 2.3e-3
 //    where the running maximum's is 1.7e-3 (128 keys, the key 4 to 8 octaves above those before
-//    it). So every probability enters as two bf16 terms (1.66e-3 there, and 2% below the
+//    it). So every probability enters as two bf16 terms (1.66e-3 there, and 4% below the
 //    running maximum on random rows), at 364 us against 324 with second terms for half of the
-//    keys, on the first case below. A block that outgrows the reference takes its score products
+//    keys, on the first case below (the other half's behind a test of whether one of them can
+//    dominate, with V read again for it: 364 as well, and 73 against 65 us for 203 tokens
+//    behind 3000). A block that outgrows the reference takes its score products
 //    twice: 2048 tokens behind 2048 in 391 us on random rows, 453 with their scores' deviation
 //    four times that, 632 where every block of every row does.
 //  * Operands are read from LDS four products ahead of their use, and the next block's loads
 //    go out between the score products.
 //
 // What bounds it: each wave reads every K and V byte of a block from LDS (64 KB a block and
-// wave at head_dim 512 for 2048 matrix-core cycles), so the 32 rows a wave holds - the most
+// wave at head_dim 512 for 3072 matrix-core cycles), so the 32 rows a wave holds - the most
 // its 512 registers allow at head_dim 512: 256 of O, 128 of Q - set the LDS traffic. With one
 // wave per SIMD at head_dim 512 the softmax between the two products is exposed. Measured, the
 // whole call with its merge, against 16 rows per wave on 16x16x32 products with V transposed

@@ -133,7 +133,8 @@ HypStatus hyp_runtime_info(HypRuntimeInfo* out);
 HypStatus hyp_device_alloc(size_t bytes, void** out_ptr);
 HypStatus hyp_device_free(void** ptr);
 /* A non-blocking HIP stream plus a 306 KiB device workspace for the calls that need one
- * (hyp_sample_greedy, hyp_sample_greedy_topk, hyp_sample_stochastic). destroy waits for the
+ * (hyp_sample_greedy, hyp_sample_greedy_topk, hyp_sample_stochastic), and from its first
+ * hyp_attention that splits a chunk's keys on the partials of those. destroy waits for the
  * device before freeing the workspace. */
 HypStatus hyp_stream_create(HypStream* out_stream);
 HypStatus hyp_stream_destroy(HypStream* stream);
