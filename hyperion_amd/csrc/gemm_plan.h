@@ -124,8 +124,8 @@ inline uint32_t filling_split(const GemmShape& g, uint64_t cus) {
 // worst, and the choice 0.7% slower than the best of the sweep on average. Ragged grids are what
 // it is for, where filling the compute units by splitting alone (filling_split, on 128-column
 // tiles for small grids) runs into a second round. Against that rule (us): down [3840, 15360]
-// 203 rows 61.3 -> 43, 700 rows 149 -> 92, 1111 rows 195 -> 136; q/k/v [8192, 3840] 300 rows 55.4
-// -> 42, 700 rows 77.2 -> 54; o [3840, 4096] 700 rows 58.5 -> 43; [15360, 3840] 300 rows 73 -> 54.
+// 203 rows 61 -> 43, 700 rows 149 -> 93, 1111 rows 195 -> 135; q/k/v [8192, 3840] 300 rows 55 ->
+// 41, 700 rows 77 -> 53; o [3840, 4096] 700 rows 59 -> 43; [15360, 3840] 300 rows 73 -> 53.
 inline GemmChoice choose_gemm(const GemmShape& g, uint64_t cus) {
     constexpr uint32_t kMaxSplits = 12u;
     const uint32_t most = filling_split(g, cus);
