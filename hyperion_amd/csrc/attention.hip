@@ -688,10 +688,12 @@ size_t attention_workspace_bytes(uint32_t n_kv_heads, uint32_t head_dim, uint32_
     return 16u * std::min<uint64_t>(blocks, kAttnMaxSplits) * n_kv_heads * row_bytes(head_dim);
 }
 
-// The chunk form: one row tile per compute unit (256 on MI355X; a plan needs no device), or
-// the decode form's rows of many kv heads.
+// The chunk form: one row tile per compute unit (256 on MI355X; a plan needs no device), with
+// more than 8 kv heads up to the two that chunk_splits can place.
 size_t attention_chunk_workspace_bytes(uint32_t n_kv_heads, uint32_t head_dim) {
-    return std::max<size_t>(256u * kChunkRows, size_t{16u} * kAttnMaxSplits * n_kv_heads) * row_bytes(head_dim);
+    constexpr size_t kRows = 256u * kChunkRows;
+    const size_t rows = std::max(kRows, size_t{16u} * kAttnMaxSplits * n_kv_heads);
+    return std::min(rows, head_dim >= 512u ? kRows : 2u * kRows) * row_bytes(head_dim);
 }
 
 bool attention_chunk_splits(const AttnArgs& a) {

@@ -164,8 +164,10 @@ uint64_t rope_table_bytes(const Geometry& g, uint32_t D) {
 
 // The attention split workspace of both layer kinds.
 uint64_t attention_ws_bytes(const Geometry& g) {
-    return std::max(hip::attention_chunk_workspace_bytes(g.kv_heads_local, g.head_dim_local),
-                    hip::attention_chunk_workspace_bytes(g.kv_heads_global, g.head_dim_global));
+    return std::max({hip::attention_chunk_workspace_bytes(g.kv_heads_local, g.head_dim_local),
+                     hip::attention_chunk_workspace_bytes(g.kv_heads_global, g.head_dim_global),
+                     hip::attention_workspace_bytes(g.kv_heads_local, g.head_dim_local, g.max_positions),
+                     hip::attention_workspace_bytes(g.kv_heads_global, g.head_dim_global, g.max_positions)});
 }
 
 }  // namespace

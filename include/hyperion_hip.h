@@ -348,9 +348,9 @@ HypStatus hyp_kv_cache_write(HypKvCache cache, const void* k, const void* v, uin
  * is read before the chunk overwrites its slots. prefix_len <= offset and <= capacity (a
  * sliding layer passes min(window, offset), a global one offset). fp32 scores and softmax,
  * P rounded to bf16 for the P.V products, output rounded to bf16. With more than 16 query rows
- * per KV head a call that splits its keys does so in partials that `stream` owns (32768 rows, or
- * 4096 per KV head, of head_dim + 2 fp32 values; made by the first such call, freed with the
- * stream), and such calls may overlap on one cache. Recorded into a graph they use none, and
+ * per KV head a call that splits its keys does so in partials that `stream` owns (32768 rows of
+ * head_dim + 2 fp32 values, up to twice as many with more than 8 KV heads below head_dim 512;
+ * made by the first such call, freed with the stream), and such calls may overlap on one cache. Recorded into a graph they use none, and
  * those of 17 to 64 query rows per KV head the handle's workspace. */
 HypStatus hyp_attention(const void* q, const void* k, const void* v, uint32_t L, uint32_t n_heads, HypKvCache cache,
                         uint32_t offset, uint32_t prefix_len, uint32_t window, void* out, HypStream stream);
