@@ -41,6 +41,22 @@ inline uint64_t row_tiles(const GemmShape& g) {   // 16-column tiles
     return t;
 }
 
+// Whether the few-row kernel takes the call. Each wave reads its rows of X from L2, about 12 TB/s
+// over the chip, so its time grows with rows x k x column tiles; the tile kernels' hardly below
+// 128 rows. Measured, the tile kernels against it (us, calls among others, weights alternating):
+//   gate + up [2 x 15360, 3840]  33 at 32 rows -> 27, but 36 -> 42 at 33
+//   [15360, 3840]                27 -> 17 at 32, 26.9 -> 24.1 at 33, 29 -> 35 at 64
+//   q/k/v [8192, 3840], o [3840, 4096]  23-25 -> 12 and 11 at 32, 19.5 and 18.3 at 64
+//   [3840, 8192]                 25.7 -> 21 at 33, 26.3 -> 25.8 at 48, 27 -> 33 at 64
+//   down [3840, 15360]           31 -> 31 at 32, 31 -> 37 at 33, 31 -> 45 at 48, 32 -> 58 at 64
+// The last line's tile calls split k, and a split call that the host waits for pays 45-55 us more
+// for its partials' allocation, which such a wait has given back: down alone 96 -> 48 at 33, 93 ->
+// 58 at 48, 92 -> 70 at 64, [3840, 8192] 85 -> 44 at 64. So: always up to 32 rows, to 64 where
+// the column tiles are at most two per compute unit.
+inline bool few_rows(const GemmShape& g, uint64_t cus) {
+    return g.m <= 32u || (g.m <= kFewRows && row_tiles(g) <= 2u * cus);
+}
+
 // As many column tiles per wave (they share its X reads) as leave 7 waves per compute unit
 // with every tile's pairs over 8 waves, then the fewest waves per tile that still do; from
 // 33 rows on at most 2 (registers, and the LDS of the sums). At 16 rows (us): [15360, 3840]
@@ -58,23 +74,6 @@ inline FewRowShape few_row_shape(const GemmShape& g, uint64_t cus) {
     uint32_t s = 1u;
     while (s < kFewWaves && tiles / nt * s < 7u * cus && 2u * s <= g.pairs) s *= 2u;
     return {nt, s};
-}
-
-// Whether the few-row kernel takes the call. Each wave reads its rows of X from L2, about 12 TB/s
-// over the chip, so its time grows with rows x k x column tiles; the tile kernels' hardly below
-// 128 rows. Measured, the tile kernels against it (us, weights alternating):
-//   gate + up [2 x 15360, 3840]  33 at 32 rows -> 27, but 36 -> 42 at 33
-//   [15360, 3840]                27 -> 17 at 32, 26.9 -> 24.1 at 33, 29 -> 35 at 64
-//   q/k/v [8192, 3840], o [3840, 4096]  23-25 -> 12 and 11 at 32, 19.5 and 18.3 at 64
-//   [3840, 8192]                 25.7 -> 21 at 33, 26.3 -> 25.8 at 48, 27 -> 30.5 at 56
-//   down [3840, 15360]           31 -> 31 at 32, but 31 -> 37 at 33, 32 -> 58 at 64
-// So: always up to 32 rows; from 33 to 64 where the column tiles are at most two per compute unit
-// and the waves read at most 200 MB of X (17 us).
-inline bool few_rows(const GemmShape& g, uint64_t cus) {
-    if (g.m <= 32u) return true;
-    if (g.m > kFewRows || row_tiles(g) > 2u * cus) return false;
-    const uint64_t reads = row_tiles(g) / few_row_shape(g, cus).tiles * g.m * g.pairs * 256u;
-    return reads <= 200'000'000u;
 }
 
 // Workgroups of one k split: (rows / tile rows) x (column tiles over the segments).

@@ -450,9 +450,8 @@ FEW_CASES = [
     (33, (2048, 16), 1088),
     (48, (4096, 2048, 2041), 256),  # 512 column tiles, the most from 33 rows on
     (64, (3840,), 704),
-    # past the kernel's bounds: 513 column tiles, and 200 MB of X read by the waves
-    (48, (4096, 2048, 2049), 256),
-    (33, (3840,), 15360),
+    (48, (4096, 2048, 2049), 256),  # 513: the 128-row tiles
+    (33, (3840,), 15360),           # three row tiles, 15 pairs a wave
 ]
 
 
