@@ -653,10 +653,11 @@ size_t row_bytes(uint32_t head_dim) { return static_cast<size_t>(head_dim) * 4u 
 
 // Key splits of the chunk form: as many as the idle compute units take (one workgroup each at
 // head_dim 512, two below), with at least 4 key blocks in each (below that the merge costs
-// more than the walk) and within the workspace. Measured unsplit and by this rule: global
-// (head_dim 512, one kv head) 203 tokens behind 3000 203 -> 57 us, 64 behind 4000 251 -> 56,
-// 1000 behind 3000 250 -> 166; sliding (256, 8 kv heads) 203 behind 700 39 -> 29, 1000
-// behind 700 50 -> 43; half as many splits as the rule gives 73-81 us on the first two.
+// more than the walk) and within the workspace. Measured unsplit (replayed from a graph) and by
+// this rule: global (head_dim 512, one kv head) 203 tokens behind 3000 250 -> 66 us, 64 behind
+// 4000 310 -> 61, 1000 behind 3000 327 -> 201; sliding (256, 8 kv heads) 203 behind 700 44 -> 30,
+// 1000 behind 700 56 -> 45. Half as many splits as the rule gives took 1.3 to 1.4 times as long
+// on the first two.
 uint32_t chunk_splits(uint32_t L, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, uint32_t keys,
                       size_t workspace_bytes) {
     const uint32_t G = n_heads / n_kv_heads;
